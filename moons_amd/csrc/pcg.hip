@@ -8,7 +8,10 @@
 // (code/handwritten/solvers/preconditioners/preconditioners.f90:55-71) and
 // modify_RHS_SF (code/handwritten/solvers/PCG/PCG_aux.f90:30-54).
 //
-// One iteration is three HBM-bound kernels over the interior cells:
+// A Jacobi solve of a grid that fits the CUs' registers and LDS (up to 128^3)
+// runs its whole loop as one resident kernel (pcg_resident.hpp).  Otherwise, in
+// a captured graph, and in the flexible PCG around the multigrid or the
+// network, one iteration is three HBM-bound kernels over the interior cells:
 //   k_pcg_matvec   q = vol*lap(p), partial (p,q)              read p, write q        16 B/cell
 //   k_pcg_update   x += a p, r -= a q, partials (r,r),(Minv r,r) read x,p,r,q write x,r 48 B/cell
 //   k_pcg_pupdate  exit test; p = b p + Minv r (+ ghosts of p)  read r,p write p        24 B/cell
@@ -38,11 +41,14 @@
 namespace moons {
 
 struct PcgCtrl {
-  int iter, done, exit_loop, iter_max, n_skip, pad_;
+  int iter, done, exit_loop, iter_max, n_skip;
+  int given_up; // the resident loop was given up (pcg_resident.hpp)
   double tol_rel, tol_abs;
   double rho[2]; // rho of the last iteration, indexed by its parity
   double alpha, beta, res0, res, mean, volsum, pq, rr, rz;
 };
+
+constexpr int kResDone = 2; // done, by a complete resident loop
 
 // ------------------------------------------------------------------ kernels
 
@@ -176,8 +182,12 @@ __global__ void __launch_bounds__(kNT) k_pcg_rhs(const double *__restrict__ b, c
 
 // Set-up exit test (PCG_solver_algorithm.f90:60-68), one block:
 // res0 = |r0|, rho = (r,z), res = sqrt|rho|; exit_loop(2) skips the loop.
-__global__ void __launch_bounds__(kNT) k_pcg_init(PcgCtrl *ctrl, const double *partB, int nb) {
+// Also empties the resident loop's slots (when given) and clears its abort word.
+__global__ void __launch_bounds__(kNT) k_pcg_init(PcgCtrl *ctrl, const double *partB, int nb,
+                                                 unsigned long long *slots, int nslots) {
   __shared__ double sh[2 * (kNT / kWave) + 2];
+  if (slots)
+    for (int q = threadIdx.x; q < nslots; q += kNT) slots[q] = q < nslots - 1 ? ~0ull : 0ull;
   double rr, rz;
   prologue_sum2<kNT>(partB, 0, partB, 1, nb, 2, sh, rr, rz);
   if (threadIdx.x == 0) {
@@ -385,6 +395,12 @@ __global__ void __launch_bounds__(kNT) k_pcg_pupdate(double *__restrict__ p, con
     }
   }
 }
+
+} // namespace moons
+
+#include "pcg_resident.hpp"
+
+namespace moons {
 
 // ----------------------------------------------------- multigrid-mode kernels
 // The FP64 flexible PCG around the FP32 V-cycle: z = V(r/vol), rho = (z,r),
@@ -603,6 +619,9 @@ struct moons_pcg_s {
   PcgCtrl *host_ctrl = nullptr; // pinned, read-backs
   PcgCtrl *host_init = nullptr; // pinned, initial control block (the source of every upload)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  ResPlan res;                  // the resident loop's box (cpt 0: the launch-per-kernel loop)
+  unsigned long long *slots = nullptr;
+  int spins = 0;                // its waits' bound
   bool noalloc = false;         // a one-shot solver over the static scratch (no host_init)
 };
 
@@ -629,7 +648,7 @@ __global__ void k_pcg_ctrl_set(PcgCtrl *ctrl, int iter_max, int n_skip, double t
                                double volsum) {
   if (threadIdx.x != 0) return;
   PcgCtrl h;
-  h.iter = h.done = h.exit_loop = h.pad_ = 0;
+  h.iter = h.done = h.exit_loop = h.given_up = 0;
   h.iter_max = iter_max;
   h.n_skip = n_skip;
   h.tol_rel = tol_rel;
@@ -683,6 +702,45 @@ static F32Map flex_map(const moons_pcg_s *S) {
 static int flex_apply(moons_pcg_s *S) {
   if (S->mg) return mg_vcycle(S->mg, &S->ctrl->done);
   return unet_prec_apply(S->unet, S->uf0, S->uz0, &S->ctrl->done);
+}
+
+template <int CPT>
+static const void *resident_fn(int op) {
+  return op == MOONS_OP_NRG_DIFFUSION ? (const void *)k_pcg_resident<kResNT, CPT, true>
+                                      : (const void *)k_pcg_resident<kResNT, CPT, false>;
+}
+static const void *resident_kernel(const ResPlan &P, int op) {
+  switch (P.cpt) {
+    case 1: return resident_fn<1>(op);
+    case 2: return resident_fn<2>(op);
+    case 4: return resident_fn<4>(op);
+    case 8: return resident_fn<8>(op);
+    default: return resident_fn<16>(op);
+  }
+}
+
+// Chooses the resident loop's box for S (Jacobi solves of a grid that fits the
+// GPU's CUs), or none.  MOONS_RESIDENT_SPINS sets the bound of its waits (0:
+// the launch-per-kernel loop), for tests of both loops and of the give-up path.
+static void resident_setup(moons_pcg_s *S) {
+  S->spins = 1 << 20;
+  if (const char *e = getenv("MOONS_RESIDENT_SPINS")) S->spins = atoi(e);
+  if (S->spins <= 0) return;
+  for (int d = 0; d < 3; ++d) // a periodic face has its partner
+    if ((S->G.bct[2 * d] == MOONS_BC_PERIODIC) != (S->G.bct[2 * d + 1] == MOONS_BC_PERIODIC)) return;
+  int dev = 0, cus = 0, per_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return;
+  const ResPlan P = resident_plan(S->G.n0, S->G.n1, S->G.n2, cus);
+  if (!P.cpt) return;
+  const void *fn = resident_kernel(P, S->op);
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kResNT, P.lds) != hipSuccess || per_cu < 1) {
+    (void)hipGetLastError();
+    return;
+  }
+  S->res = P;
 }
 
 static NrgK nrg_k(const moons_pcg_s *S) {
@@ -808,6 +866,13 @@ int moons_pcg_sf_create(moons_mesh_t m, int op, int prec, moons_field_t x, moons
     moons_pcg_destroy(S);
     return fail(MOONS_ERR_HIP, "moons_pcg_sf_create: allocation failed");
   }
+  if (prec != MOONS_PREC_MG_FP32) {
+    resident_setup(S);
+    if (S->res.cpt && hipMalloc(&S->slots, kResSlotWords * sizeof(unsigned long long)) != hipSuccess) {
+      moons_pcg_destroy(S);
+      return fail(MOONS_ERR_HIP, "moons_pcg_sf_create: allocation failed");
+    }
+  }
   std::memset(S->host_init, 0xff, sizeof(PcgCtrl)); // differs from any real block: first upload writes it
   (void)hipMemsetAsync(S->r, 0, bytes, stream());
   (void)hipMemsetAsync(S->p, 0, bytes, stream());
@@ -891,6 +956,7 @@ int moons_pcg_destroy(moons_pcg_t S) {
   double *bufs[] = {S->r, S->p, S->q, S->partA, S->partB, S->partM, S->partC, S->kf[0], S->kf[1], S->kf[2]};
   for (double *b : bufs)
     if (b) (void)hipFree(b);
+  if (S->slots) (void)hipFree(S->slots);
   if (S->ctrl) (void)hipFree(S->ctrl);
   if (S->host_ctrl) (void)hipHostFree(S->host_ctrl);
   if (S->host_init) (void)hipHostFree(S->host_init);
@@ -937,6 +1003,24 @@ int moons_pcg_set_isp(moons_pcg_t S, int iter_max, double tol_rel, double tol_ab
 
 
 
+// The whole loop in one kernel, then x and its BCs; host_ctrl holds the result
+// (given_up: x's cells are unchanged).
+static int pcg_solve_resident(moons_pcg_s *S, moons_field_t x) {
+  const ResPlan &P = S->res;
+  NrgK K = nrg_k(S);
+  const double *xd = x->d;
+  int by = P.by, gy = P.gy, spins = S->spins;
+  void *args[] = {(void *)&xd, &S->r, &S->p, &S->q, &S->G, &by, &gy, &S->ctrl, &S->slots, &spins, &K};
+  MOONS_HIP(hipLaunchKernel(resident_kernel(P, S->op), dim3(P.nb()), dim3(kResNT), args, P.lds, stream()));
+  hipLaunchKernelGGL(k_pcg_take, dim3(S->G.nblocks), dim3(kNT), 0, stream(), x->d, S->q, S->G, S->ctrl, S->slots);
+  MOONS_LAUNCH_CHECK();
+  int st = launch_apply_bcs(x, false);
+  if (st) return st;
+  MOONS_HIP(hipMemcpyAsync(S->host_ctrl, S->ctrl, sizeof(PcgCtrl), hipMemcpyDeviceToHost, stream()));
+  MOONS_HIP(hipStreamSynchronize(stream()));
+  return MOONS_OK;
+}
+
 static int pcg_solve_impl(moons_pcg_s *S, moons_field_t x, moons_field_t b) {
   int st = pcg_upload_ctrl(S);
   if (st) return st;
@@ -952,8 +1036,20 @@ static int pcg_solve_impl(moons_pcg_s *S, moons_field_t x, moons_field_t b) {
     else
       hipLaunchKernelGGL((k_pcg_rhs<false, false>), grid, block, 0, stream(), b->d, x->d, S->r, S->p, S->G, S->ctrl,
                          S->partM, S->partB, alln, (float *)nullptr, flex_map(S), nrg_k(S));
-    hipLaunchKernelGGL(k_pcg_init, dim3(1), block, 0, stream(), S->ctrl, S->partB, S->G.nblocks);
+    const bool resident = S->res.cpt && !sync_free();
+    hipLaunchKernelGGL(k_pcg_init, dim3(1), block, 0, stream(), S->ctrl, S->partB, S->G.nblocks,
+                       resident ? S->slots : nullptr, (int)kResSlotWords);
     MOONS_LAUNCH_CHECK();
+    if (resident) {
+      if ((st = pcg_solve_resident(S, x))) return st;
+      if (!S->host_ctrl->given_up) return MOONS_OK;
+      // not every block was resident: the solve again from x, a kernel at a time
+      const ResPlan keep = S->res;
+      S->res.cpt = 0;
+      st = pcg_solve_impl(S, x, b);
+      S->res = keep;
+      return st;
+    }
   } else {
     // z0 = V(r0/vol), rho0 = (z0,r0), p = z0
     hipLaunchKernelGGL((k_pcg_rhs<true, false>), grid, block, 0, stream(), b->d, x->d, S->r, S->p, S->G, S->ctrl,
@@ -1307,6 +1403,9 @@ int moons_pcg_sf_solve_noalloc(moons_field_t x, moons_field_t b, int iter_max, d
   S.r = S.partC + 2 * kNaBlocks;
   S.p = S.r + kNaCells;
   S.q = S.p + kNaCells;
+  static_assert(kResSlotWords <= 2 * kNaBlocks, "the resident loop's slots do not fit the scratch");
+  resident_setup(&S);
+  S.slots = reinterpret_cast<unsigned long long *>(S.partC); // the multigrid's sums, unused here
   PcgCtrl hc;
   std::memset(&hc, 0, sizeof hc);
   S.host_ctrl = &hc;
