@@ -223,7 +223,14 @@ __global__ void __launch_bounds__(256) k_mg_smooth(LevelDev L, int color, int ze
 // the 8 XCDs) sweeps a contiguous slab of planes q, whose neighbouring blocks
 // share its L2: the other colour's x read by the planes q - 1, q, q + 1 and
 // both halves of a 128-byte row are then fetched from HBM once.
-constexpr int kLineMax = 128; // longest line (at least 16 lines per block)
+// Longest line.  A stretched level whose lines are longer smooths by points,
+// which damp the error along the stretched direction badly: with lines up to
+// 128 cells the 256^3 channel took 28 iterations of a 545 us V-cycle, 30.2 ms;
+// with lines of 256 it takes 13 of 671 us, 16.7 ms, to a smaller error.
+// Such a line is 32 threads of 8 cells, 16 lines a block of 512: 21.9 us a
+// half-sweep at 256^3 (blocks of 1024 28.6, of 256 29.2; 16 cells a thread
+// 23.2 and 24.7), against 100 MB at 4.4 TB/s.
+constexpr int kLineMax = 256;
 constexpr long long kLineMinCells = 32LL * 32 * 32; // levels this small smooth by points
 // MOONS_MG_LINE_MIN_CELLS overrides kLineMinCells, for tuning runs.
 static long long line_min_cells() {
@@ -251,7 +258,7 @@ __device__ __forceinline__ float3 line_row(const LevelDev &L, int i, int m, int 
   const int ic = ok ? i : 1, mc = ok ? m : 0, tc = t < nl ? t : nl - 1;
   const int j = D == 1 ? tc + 1 : q, k = D == 1 ? q : tc + 1;
   // plane offsets: h0 (j - 1) and h0 n1 (k - 1), one of them block-uniform;
-  // every factor is below 2^24 (lines of at most 128 cells, levels below 2^30)
+  // every factor is below 2^24 (lines of at most 256 cells, levels below 2^30)
   const int h0 = L.h0, hn = L.h0 * L.n1;
   const int oj = (int)__umul24((unsigned)h0, (unsigned)(j - 1)), ok_ = (int)__umul24((unsigned)hn, (unsigned)(k - 1));
   const int col = (ic + j + k) & 1;
@@ -1333,6 +1340,7 @@ static void line_half_d(const LevelDev &L, int c, bool zero_guess, const int *do
   if (nl <= 16) line_launch<D, 16, 64, 4>(L, c, zg, done, o);
   else if (nl <= 32) line_launch<D, 32, 128, 4>(L, c, zg, done, o);
   else if (nl <= 64) line_launch<D, 64, 128, 4>(L, c, zg, done, o);
+  else if (nl <= 128) line_launch<D, 128, 512, 8>(L, c, zg, done, o);
   else line_launch<D, kLineMax, 512, 8>(L, c, zg, done, o);
 }
 
@@ -1470,6 +1478,19 @@ int mg_vcycle(MGHier *h, const int *done) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MOONS_ERR_HIP, std::string("multigrid launch: ") + hipGetErrorString(e));
   return MOONS_OK;
+}
+
+// The share of the solver's relative tolerance that a solve with this
+// preconditioner goes on to.  Lines longer than 128 cells take out the rough
+// part of the error, which the residual weighs most, so that at one residual
+// the error left is up to 14 times the one that point sweeps leave (14 grids
+// with 136 to 192 cells along y or z: 0.5 to 14 times at 1e-8).  A tenth of the
+// tolerance still leaves 0.05 to 1.4 times it; a twentieth, 2 to 6 iterations
+// more than the tolerance itself, less than it on every one of them.
+double mg_stop_factor(const MGHier *h) {
+  for (const LevelDev &L : h->L)
+    if ((L.line1 && L.n1 > 128) || (L.line2 && L.n2 > 128)) return 0.05;
+  return 1.0;
 }
 
 void mg_begin_solve(MGHier *h) { h->cycle = 0; }

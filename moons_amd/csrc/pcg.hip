@@ -44,6 +44,7 @@ struct PcgCtrl {
   int iter, done, exit_loop, iter_max, n_skip;
   int given_up; // the resident loop was given up (pcg_resident.hpp)
   double tol_rel, tol_abs;
+  double tol_stop; // the relative residual the loop goes on to: tol_rel, or less (mg_stop_factor)
   double rho[2]; // rho of the last iteration, indexed by its parity
   double alpha, beta, res0, res, mean, volsum, pq, rr, rz;
 };
@@ -327,7 +328,7 @@ __device__ __forceinline__ ExitDecision exit_decision(const PcgCtrl *ctrl, int i
     e.res = sqrt(fabs(rr));
     const bool e1 = e.res / ctrl->res0 < ctrl->tol_rel, e2 = e.res < ctrl->tol_abs, e3 = it >= ctrl->iter_max;
     e.flags = (e1 ? 1 : 0) | (e2 ? 2 : 0) | (e3 ? 4 : 0);
-    e.stop = e1 || e2 || e3;
+    e.stop = e.res / ctrl->res0 < ctrl->tol_stop || e2 || e3;
   }
   if (!e.stop && it >= ctrl->iter_max) {
     e.flags |= 4;
@@ -651,13 +652,15 @@ __global__ void k_pcg_ctrl_set(PcgCtrl *ctrl, int iter_max, int n_skip, double t
   h.iter = h.done = h.exit_loop = h.given_up = 0;
   h.iter_max = iter_max;
   h.n_skip = n_skip;
-  h.tol_rel = tol_rel;
+  h.tol_rel = h.tol_stop = tol_rel;
   h.tol_abs = tol_abs;
   h.rho[0] = h.rho[1] = 0.0;
   h.alpha = h.beta = h.res0 = h.res = h.mean = h.pq = h.rr = h.rz = 0.0;
   h.volsum = volsum;
   *ctrl = h;
 }
+
+static double tol_stop(const moons_pcg_s *S) { return S->tol_rel * (S->mg ? mg_stop_factor(S->mg) : 1.0); }
 
 // The initial control block lives in its own pinned buffer, written only
 // here, so a captured copy of it replays the same values.
@@ -673,6 +676,7 @@ static int pcg_upload_ctrl(moons_pcg_s *S) {
   h.iter_max = S->iter_max;
   h.n_skip = S->n_skip;
   h.tol_rel = S->tol_rel;
+  h.tol_stop = tol_stop(S);
   h.tol_abs = S->tol_abs;
   h.volsum = S->volsum;
   if (std::memcmp(&h, S->host_init, sizeof(PcgCtrl)) != 0) {
@@ -1086,7 +1090,7 @@ static int pcg_solve_impl(moons_pcg_s *S, moons_field_t x, moons_field_t b) {
       tail_pending = false;
     }
     int chunk = launched == 0 ? (mg ? 3 : 16)
-                              : next_chunk(*S->host_ctrl, S->tol_rel, mg ? 1 : 4, mg ? 32 : 512);
+                              : next_chunk(*S->host_ctrl, tol_stop(S), mg ? 1 : 4, mg ? 32 : 512);
     chunk = std::min(chunk, S->iter_max - launched);
     for (int c = 0; c < chunk; ++c) {
       const int it = launched + c + 1;

@@ -183,7 +183,7 @@ class Level:
 
 COARSE_CELLS = 4  # a level of at most this many cells per direction is the coarsest
 LINE_MIN_CELLS = 32 * 32 * 32  # levels of at most this many cells are smoothed by points
-LINE_MAX = 128  # longest line the device holds in LDS
+LINE_MAX = 256  # longest line the device holds in LDS
 
 
 def build(hn3, bct, max_levels=16, coarse_cells=COARSE_CELLS):

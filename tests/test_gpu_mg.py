@@ -202,6 +202,61 @@ def test_vcycle_ragged_lines_match_restatement(gpu, case):
     assert P.mg_info()[0] == len(levels)
 
 
+LONG = {  # lines of 129 to 256 cells: the slot full, one cell over the shorter slot, ragged
+    "x12_y256_z12": ((12, 256, 12), [3, 3, 2, 2, 2, 1]),
+    "x16_y16_z130": ((16, 16, 130), [2, 2, 1, 2, 2, 2]),
+    "x8_y200_z24": ((8, 200, 24), [2, 1, 2, 1, 1, 1]),
+}
+
+
+def restated_in_fp32(levels, f, bct, monkeypatch):
+    """The restatement's V-cycle with every array in FP32."""
+    for L in levels:
+        for name in ("wm", "wp", "dg"):
+            setattr(L, name, [a.astype(np.float32) for a in getattr(L, name)])
+
+    class Single:
+        def __getattr__(self, name):
+            return getattr(np, name)
+
+        def zeros(self, shape):
+            return np.zeros(shape, dtype=np.float32)
+
+    with monkeypatch.context() as mp:
+        mp.setattr(MGO, "np", Single())
+        return MGO.vcycle(levels, f.astype(np.float32), bct)
+
+
+@pytest.mark.parametrize("case", list(LONG))
+def test_vcycle_long_lines_match_restatement(gpu, monkeypatch, case):
+    """Zebra lines longer than 128 cells against the restatement, which solves
+    each line by elimination.  The longer the stretched line, the worse the
+    system's condition, so the bound is the restatement's own error when it is
+    evaluated in FP32 (3.8e-5 for 256 cells, 6.5e-6 for 130), times 4 for
+    another order of the same roundings."""
+    (nx, ny, nz), bct = LONG[case]
+    print(f"vcycle long lines {case}", flush=True)
+    hs = [O.uniform_nodes(0.0, 1.0, nx), O.roberts_both_nodes(0.0, 1.0, ny, 1.05),
+          O.roberts_both_nodes(0.0, 1.0, nz, 1.05)]
+    g, m = O.Grid(*hs), gpu.mesh(*hs)
+    levels = MGO.build(hs, bct)
+    assert levels[0].line_dirs == [1, 2]
+    x = gpu.SF(m, "CC").set_BCs([NAMES[t] for t in bct], None, all_Neumann=(1 not in bct))
+    P = mg_solver(gpu, m, x)
+    r = np.zeros(g.shape(0), order="F")
+    r[1:-1, 1:-1, 1:-1] = np.random.default_rng(17).standard_normal((nx, ny, nz))
+    Z = gpu.SF(m, "CC")
+    P.apply_prec(gpu.SF(m, "CC").upload(r), Z)
+    vol = O.volume(g, 0)
+    f = np.zeros(g.shape(0))
+    f[1:-1, 1:-1, 1:-1] = r[1:-1, 1:-1, 1:-1] / vol[1:-1, 1:-1, 1:-1]
+    z, zr, z32 = (a[1:-1, 1:-1, 1:-1] for a in (Z.download(), MGO.vcycle(levels, f, bct),
+                                                restated_in_fp32(MGO.build(hs, bct), f, bct, monkeypatch)))
+    err, own = (np.linalg.norm(a - zr) / np.linalg.norm(zr) for a in (z, z32))
+    print(f"device {err:.2e}, restatement in FP32 {own:.2e}", flush=True)
+    assert err < 4 * own, (err, own)
+
+
 @pytest.mark.parametrize("case", list(CASES))
 def test_mixed_pcg_matches_fp64_oracle(gpu, case):
     N, beta, bct = CASES[case]

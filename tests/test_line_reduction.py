@@ -73,3 +73,7 @@ def test_line_order_matches_dense_solve(NP, C):
         ref = np.linalg.solve(M, d)
         x = emulate(a, c, d, NP, C)
         assert np.max(np.abs(x - ref)) <= 1e-12 * np.max(np.abs(ref)), (NP, C, nl)
+
+
+def test_line_order_of_the_longest_slot():
+    test_line_order_matches_dense_solve(256, 8)
