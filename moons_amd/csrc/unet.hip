@@ -13,8 +13,8 @@
 // implicit GEMM: M = voxels (16 per MFMA tile), N = output channels, K = 27
 // taps x input channels; v_mfma_f32_16x16x16_bf16 with A = 16 voxels x 16
 // input channels (one 8-byte load per lane), B = weights pre-packed in
-// fragment order.  Layers with 4 input or 1 output channel are plain FP32
-// kernels (0.4% of the flops).
+// fragment order.  The 4-channel input layer packs
+// 8 taps into a 16x16x32 MFMA; the 1-channel output layer is a plain FP32 kernel.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -286,48 +286,110 @@ __global__ void __launch_bounds__(kUT) k_conv_reduce(const float *__restrict__ P
 }
 
 // dW partials: part[chunk][tap][ci][co] = sum over the chunk's voxels of
-// X[v + tap][ci] * dY[v][co] (MFMA with M = ci, N = co, K = voxels).
-template <int NB>
+// X[v + tap][ci] * dY[v][co] (MFMA with M = ci, N = co, K = 16 voxels).  A wave
+// takes the three taps of one (dz, dy) row.  ROWS: n0 is a multiple of 4, so a
+// lane's four voxels are neighbours in x and the six values of its channel at
+// x - 1 .. x + 4 serve all three taps; with dY loaded once that is 10 loads
+// for three MFMAs where a wave a tap took 24.  (A coarse level's n0 may be any
+// number: then each voxel has its own loads.)  The loads of the next 16 voxels
+// are issued before the products of the present ones.
+template <int NB, bool ROWS>
 __global__ void __launch_bounds__(64) k_conv_dw(const bf16 *__restrict__ X, int Cin, const bf16 *__restrict__ dY,
                                                int n0, int n1, int n2, int chunk, float *__restrict__ part) {
   const int lane = threadIdx.x;
   const int c = blockIdx.x;
   const int KB = Cin >> 4;
-  const int tap = blockIdx.y / KB, kb = blockIdx.y % KB;
+  const int row = blockIdx.y / KB, kb = blockIdx.y % KB;
   const int nvox = n0 * n1 * n2;
   const int s0 = n0 + 2, s1 = n1 + 2;
-  const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const int off = (dz * s1 + dy) * s0 + dx;
+  const int off = ((row / 3 - 1) * s1 + (row % 3 - 1)) * s0;
   const int Cout = NB * 16;
-  f32x4 acc[NB];
+  f32x4 acc[3][NB];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int e = 0; e < 3; ++e)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[e][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int v0 = c * chunk, v1 = min(nvox, v0 + chunk);
-  const int ci = kb * 16 + (lane & 15);
-  for (int vs = v0; vs < v1; vs += 16) {
-    s16x4 a;
+  const bf16 *Xc = X + kb * 16 + (lane & 15), *Yc = dY + (lane & 15);
+  constexpr int XE = ROWS ? 6 : 12;
+  bf16 xn[XE], yn[NB][4];
+  auto load = [&](int vs) {
+    const int v = vs + (lane >> 4) * 4;
     int pv[4];
     bool ok[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int v = vs + (lane >> 4) * 4 + j;
-      ok[j] = v < v1;
-      pv[j] = pvox(ok[j] ? v : 0, n0, n1);
-      a[j] = ok[j] ? (short)X[(size_t)(pv[j] + off) * Cin + ci] : (short)0;
+    for (int j = 0; j < 4; ++j) { // ROWS: v1 is a multiple of 4, the four are all inside or all past it
+      ok[j] = ROWS && j > 0 ? ok[0] : v + j < v1;
+      pv[j] = ROWS && j > 0 ? pv[0] + j : pvox(ok[j] ? v + j : 0, n0, n1);
     }
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      s16x4 b;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ok[j] ? (short)dY[(size_t)pv[j] * Cout + nb * 16 + (lane & 15)] : (short)0;
-      acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[nb], 0, 0, 0);
+    for (int e = 0; e < XE; ++e) {
+      const int at = ROWS ? pv[0] + off + e - 1 : pv[e & 3] + off + (e >> 2) - 1;
+      xn[e] = ok[ROWS ? 0 : e & 3] ? Xc[(size_t)at * Cin] : (bf16)0;
     }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) yn[nb][j] = ok[j] ? Yc[(size_t)pv[j] * Cout + nb * 16] : (bf16)0;
+  };
+  load(v0);
+  for (int vs = v0; vs < v1; vs += 16) {
+    s16x4 a[3], b[NB];
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[e][j] = (short)xn[ROWS ? e + j : 4 * e + j];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[nb][j] = (short)yn[nb][j];
+    if (vs + 16 < v1) load(vs + 16);
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[e][nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[e], b[nb], acc[e][nb], 0, 0, 0);
   }
-  float *out = part + ((size_t)c * 27 + tap) * Cin * Cout;
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+  for (int e = 0; e < 3; ++e) {
+    float *out = part + ((size_t)c * 27 + row * 3 + e) * Cin * Cout;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) out[(size_t)(kb * 16 + (lane >> 4) * 4 + j) * Cout + nb * 16 + (lane & 15)] = acc[nb][j];
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        out[(size_t)(kb * 16 + (lane >> 4) * 4 + j) * Cout + nb * 16 + (lane & 15)] = acc[e][nb][j];
+  }
+}
+
+// The same for the 4-channel input layer: the M rows are the three taps of the
+// (dz, dy) row times the 4 channels (12 of 16 used), N the 16 output channels.
+// Vector sums of 64 products a voxel took 59 us at 32^3 (77 with their block
+// trees), this 12.
+__global__ void __launch_bounds__(64) k_conv_dw_in(const bf16 *__restrict__ X, const bf16 *__restrict__ dY, int n0,
+                                                  int n1, int n2, int chunk, float *__restrict__ part) {
+  const int lane = threadIdx.x, c = blockIdx.x, row = blockIdx.y;
+  const int nvox = n0 * n1 * n2, s0 = n0 + 2, s1 = n1 + 2;
+  const int e = (lane & 15) >> 2, ci = lane & 3;
+  const int off = ((row / 3 - 1) * s1 + (row % 3 - 1)) * s0 + min(e, 2) - 1;
+  const int v0 = c * chunk, v1 = min(nvox, v0 + chunk);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int vs = v0; vs < v1; vs += 16) {
+    const int v = vs + (lane >> 4) * 4;
+    const bool ok = v < v1;
+    const int pv = pvox(ok ? v : 0, n0, n1);
+    s16x4 a, b;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[j] = ok && e < 3 ? (short)X[(size_t)(pv + j + off) * 4 + ci] : (short)0;
+      b[j] = ok ? (short)dY[(size_t)(pv + j) * 16 + (lane & 15)] : (short)0;
+    }
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+  }
+  // D row 4 (lane / 16) + j: tap lane / 16, channel j
+  if (lane < 48) {
+    float *out = part + ((size_t)c * 27 + row * 3 + (lane >> 4)) * 64;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j * 16 + (lane & 15)] = acc[j];
+  }
 }
 
 // dW (+)= sum over chunks of the partials, in chunk order
@@ -335,77 +397,137 @@ __global__ void __launch_bounds__(kUT) k_reduce_chunks(const float *part, int nc
   const size_t t = (size_t)blockIdx.x * kUT + threadIdx.x;
   if (t >= n) return;
   float s = 0.f;
+#pragma unroll 8
   for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * n + t];
   dW[t] = accumulate ? dW[t] + s : s;
 }
 
-// db (+)= sum over voxels of dY[v][co]; one block per output channel
-__global__ void __launch_bounds__(kUT) k_dbias(const bf16 *dY, int C, int n0, int n1, int n2, float *db, int accumulate) {
-  __shared__ float sh[kUT];
-  const int co = blockIdx.x;
+// Bias gradient partials: part[block][co] = sum over the block's chunk of
+// voxels of dY[v][co]; k_reduce_chunks adds the blocks.  A thread owns 8
+// channels (one 16-byte load a voxel) of every (kUT / (C / 8))-th voxel.  One
+// block a channel over all voxels, as this was, left 16 blocks with 2-byte
+// loads and one accumulation chain each: 48 us at 32^3, now 5 us with the sum.
+__global__ void __launch_bounds__(kUT) k_dbias_part(const bf16 *__restrict__ dY, int C, int n0, int n1, int n2,
+                                                   int chunk, float *__restrict__ part) {
+  __shared__ float sh[kUT][9];
+  const int C8 = C / 8, lanes = kUT / C8, cg = threadIdx.x % C8, lane = threadIdx.x / C8;
   const int nvox = n0 * n1 * n2;
-  float s = 0.f;
-  for (int v = threadIdx.x; v < nvox; v += kUT) s += bf2f(dY[(size_t)pvox(v, n0, n1) * C + co]);
-  sh[threadIdx.x] = s;
+  const int v0 = blockIdx.x * chunk, v1 = min(nvox, v0 + chunk);
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (lane < lanes) // (C / 8 need not divide the block)
+    for (int v = v0 + lane; v < v1; v += lanes) {
+      const u16x8 q = *reinterpret_cast<const u16x8 *>(dY + (size_t)pvox(v, n0, n1) * C + cg * 8);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] += bf2f(q[j]);
+    }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) sh[threadIdx.x][j] = a[j];
   __syncthreads();
-  for (int w = kUT / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x < C) {
+    float r = 0.f;
+    for (int l = 0; l < lanes; ++l) r += sh[l * C8 + threadIdx.x / 8][threadIdx.x % 8];
+    part[(size_t)blockIdx.x * C + threadIdx.x] = r;
   }
-  if (threadIdx.x == 0) db[co] = accumulate ? db[co] + sh[0] : sh[0];
 }
 
 // ------------------------------------------------------ small-channel layers
-// first layer: Y[v][0..15] = relu(b + sum_tap,ci W[tap][ci][co] X[v+tap][ci]), Cin = 4
-__global__ void __launch_bounds__(kUT) k_conv_in(const bf16 *__restrict__ X, const float *__restrict__ W,
+// first layer: Y[v][0..15] = relu(b + sum_tap,ci W[tap][ci][co] X[v+tap][ci]), Cin = 4,
+// as an implicit GEMM with K = 27 taps x 4 channels = 108 padded to 128: four
+// v_mfma_f32_16x16x32_bf16 per 16 voxels (the input and the weights are BF16
+// values, so the products are exact and the sums FP32).  Lane l holds the 8
+// channels of taps 8 s + 2 (l / 16) and the next one in step s: two 8-byte
+// loads.  WB: k_pack_in's fragments.  A thread a voxel and channel on the
+// vector units spent 118 us at 64^3 (half a billion FP32 multiplications
+// behind 2-value loads); this takes 15.
+constexpr int kInGroups = 4; // 16-voxel groups a wave
+__global__ void __launch_bounds__(kUT) k_conv_in(const bf16 *__restrict__ X, const u16x8 *__restrict__ WB,
                                                 const float *__restrict__ bias, bf16 *__restrict__ Y, int n0, int n1,
                                                 int n2, const int *done) {
-  // a thread per voxel and output channel (the channel fastest: the 16
-  // threads of a voxel share its input loads and store 32 contiguous bytes)
   if (gated(done)) return;
-  const int t = blockIdx.x * kUT + threadIdx.x;
-  const int v = t >> 4, co = t & 15;
-  if (v >= n0 * n1 * n2) return;
-  const int s0 = n0 + 2, s1 = n1 + 2;
-  const int pv = pvox(v, n0, n1);
-  float acc = bias[co];
-  for (int tap = 0; tap < 27; ++tap) {
-    const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-    // the voxel's 4 channels in one 8-byte load
-    const uint2 q = *reinterpret_cast<const uint2 *>(X + (size_t)(pv + (dz * s1 + dy) * s0 + dx) * 4);
-    const unsigned qw[2] = {q.x, q.y};
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nvox = n0 * n1 * n2;
+  const int base = (blockIdx.x * (kUT / 64) + wave) * 16 * kInGroups;
+  if (base >= nvox) return;
+  const int s0 = n0 + 2, s1 = n1 + 2, co = lane & 15;
+  u16x8 b[4];
+  int off[4][2];
+  bool live[4][2];
 #pragma unroll
-    for (int ci = 0; ci < 4; ++ci) {
-      const float xv = __uint_as_float((ci & 1) ? (qw[ci >> 1] & 0xFFFF0000u) : (qw[ci >> 1] << 16));
-      acc += xv * W[(tap * 4 + ci) * 16 + co];
+  for (int s = 0; s < 4; ++s) {
+    b[s] = WB[s * 64 + lane];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int tap = 8 * s + 2 * (lane >> 4) + h;
+      live[s][h] = tap < 27;
+      const int tc = live[s][h] ? tap : 13;
+      off[s][h] = ((tc / 9 - 1) * s1 + ((tc / 3) % 3 - 1)) * s0 + tc % 3 - 1;
     }
   }
-  Y[(size_t)pv * 16 + co] = f2bf(fmaxf(acc, 0.f));
+  const float bv = bias[co];
+#pragma unroll
+  for (int g = 0; g < kInGroups; ++g) {
+    const int v = base + g * 16 + co;
+    const int pv = pvox(v < nvox ? v : 0, n0, n1);
+    f32x4 acc = f32x4{bv, bv, bv, bv};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      uint2 q[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        q[h] = *reinterpret_cast<const uint2 *>(X + (size_t)(pv + off[s][h]) * 4);
+        if (!live[s][h]) q[h] = make_uint2(0u, 0u);
+      }
+      const uint4 a = make_uint4(q[0].x, q[0].y, q[1].x, q[1].y);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b[s]), acc,
+                                                    0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int w = base + g * 16 + (lane >> 4) * 4 + j;
+      if (w < nvox) Y[(size_t)pvox(w, n0, n1) * 16 + co] = f2bf(fmaxf(acc[j], 0.f));
+    }
+  }
 }
 
 // last layer: out[pv] = scale * (b + sum_ci sum_tap W[tap][ci] X[v+tap][ci]),
-// Cin = 16, FP32 padded output.  16 threads a voxel, one per input channel,
-// each summing its channel over the taps; the 16 sums are added in a fixed
-// butterfly (deterministic) and lane ci = 0 writes.
+// Cin = 16, FP32 padded output.  A block owns a 16 x 4 x 4 voxel tile, stages
+// its halo (18 x 6 x 6 voxels) in LDS once, as two arrays of 8 channels so
+// that neighbouring voxels' 16-byte words are neighbours, and a thread sums
+// one voxel; the weights are the same for every lane.  With a thread a voxel
+// and channel, each input was read 27 times through L2 by 2-byte loads: 41 us
+// at 64^3, now 13.
+constexpr int kOX = 16, kOY = 4, kOZ = 4;
 __global__ void __launch_bounds__(kUT) k_conv_out(const bf16 *__restrict__ X, const float *__restrict__ W,
                                                  const float *__restrict__ bias, float *__restrict__ out, int n0, int n1,
                                                  int n2, const float *scale, const int *done) {
   if (gated(done)) return;
-  const int t = blockIdx.x * kUT + threadIdx.x;
-  const int v = t >> 4, ci = t & 15;
-  const bool live = v < n0 * n1 * n2;
-  const int s0 = n0 + 2, s1 = n1 + 2;
-  const int pv = pvox(live ? v : 0, n0, n1);
-  float acc = 0.f;
-  for (int tap = 0; tap < 27; ++tap) {
-    const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-    acc += bf2f(X[(size_t)(pv + (dz * s1 + dy) * s0 + dx) * 16 + ci]) * W[tap * 16 + ci];
+  constexpr int HX = kOX + 2, HY = kOY + 2, HZ = kOZ + 2, NH = HX * HY * HZ;
+  __shared__ u16x8 sx[2][NH];
+  const int x0 = blockIdx.x * kOX, y0 = blockIdx.y * kOY, z0 = blockIdx.z * kOZ;
+  const int s0 = n0 + 2, s1 = n1 + 2, s2 = n2 + 2;
+  for (int q = threadIdx.x; q < 2 * NH; q += kUT) {
+    const int v = q >> 1, w = q & 1;
+    // (cells past the grid's edge repeat its last ones and are not used)
+    const int hx = min(x0 + v % HX, s0 - 1), hy = min(y0 + (v / HX) % HY, s1 - 1), hz = min(z0 + v / (HX * HY), s2 - 1);
+    sx[w][v] = *reinterpret_cast<const u16x8 *>(X + (((size_t)hz * s1 + hy) * s0 + hx) * 16 + w * 8);
   }
+  __syncthreads();
+  const int tx = threadIdx.x % kOX, ty = (threadIdx.x / kOX) % kOY, tz = threadIdx.x / (kOX * kOY);
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 16);
-  if (live && ci == 0) {
-    const float r = bias[0] + acc;
-    out[pv] = scale ? r * (*scale) : r;
+  for (int tap = 0; tap < 27; ++tap) {
+    const int at = ((tz + tap / 9) * HY + ty + (tap / 3) % 3) * HX + tx + tap % 3;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const u16x8 q = sx[w][at];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j & 3] = fmaf(bf2f(q[j]), W[tap * 16 + w * 8 + j], acc[j & 3]);
+    }
+  }
+  const int i = x0 + tx, j = y0 + ty, k = z0 + tz;
+  if (i < n0 && j < n1 && k < n2) {
+    const float r = bias[0] + ((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    out[((size_t)(k + 1) * s1 + (j + 1)) * s0 + i + 1] = scale ? r * (*scale) : r;
   }
 }
 
@@ -430,46 +552,44 @@ __global__ void __launch_bounds__(kUT) k_conv_out_dx(const float *__restrict__ d
   for (int ci = 0; ci < 16; ++ci) dX[(size_t)pv * 16 + ci] = f2bf(acc[ci]);
 }
 
-// small-channel dW partials (first and last layers): one block per (chunk, tap),
-// each thread a voxel range, CI x CO sums reduced across the block.
-// X: CI channels BF16; G: CO channels, BF16 (gb) or FP32 padded scalar (gf, CO = 1).
-template <int CI, int CO>
-__global__ void __launch_bounds__(kUT) k_small_dw(const bf16 *__restrict__ X, const bf16 *__restrict__ gb,
-                                                 const float *__restrict__ gf, int n0, int n1, int n2, int chunk,
-                                                 float *__restrict__ part) {
-  __shared__ float sh[kUT];
+// dW partials of the output layer (16 -> 1): one block per (chunk, tap), each
+// thread a voxel range, its 16 sums added over the wave by shuffles, then over
+// the waves.  G: the FP32 padded output gradient.
+__global__ void __launch_bounds__(kUT) k_out_dw(const bf16 *__restrict__ X, const float *__restrict__ G, int n0, int n1,
+                                               int n2, int chunk, float *__restrict__ part) {
+  __shared__ float sh[kUT / 64][16];
   const int c = blockIdx.x, tap = blockIdx.y;
   const int nvox = n0 * n1 * n2;
   const int s0 = n0 + 2, s1 = n1 + 2;
-  const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const int off = (dz * s1 + dy) * s0 + dx;
-  float acc[CI * CO];
+  const int off = ((tap / 9 - 1) * s1 + ((tap / 3) % 3 - 1)) * s0 + tap % 3 - 1;
+  float acc[16];
 #pragma unroll
-  for (int q = 0; q < CI * CO; ++q) acc[q] = 0.f;
+  for (int q = 0; q < 16; ++q) acc[q] = 0.f;
   const int v0 = c * chunk, v1 = min(nvox, v0 + chunk);
   for (int v = v0 + threadIdx.x; v < v1; v += kUT) {
     const int pv = pvox(v, n0, n1);
-    float g[CO];
+    const float g = G[pv];
+    const u16x8 *x = reinterpret_cast<const u16x8 *>(X + (size_t)(pv + off) * 16);
+    const u16x8 lo = x[0], hi = x[1];
 #pragma unroll
-    for (int co = 0; co < CO; ++co) g[co] = gf ? gf[pv] : bf2f(gb[(size_t)pv * CO + co]);
-#pragma unroll
-    for (int ci = 0; ci < CI; ++ci) {
-      const float xv = bf2f(X[(size_t)(pv + off) * CI + ci]);
-#pragma unroll
-      for (int co = 0; co < CO; ++co) acc[ci * CO + co] += xv * g[co];
+    for (int q = 0; q < 8; ++q) {
+      acc[q] += bf2f(lo[q]) * g;
+      acc[8 + q] += bf2f(hi[q]) * g;
     }
   }
-  float *out = part + ((size_t)c * 27 + tap) * CI * CO;
 #pragma unroll
-  for (int q = 0; q < CI * CO; ++q) {
-    sh[threadIdx.x] = acc[q];
-    __syncthreads();
-    for (int w = kUT / 2; w > 0; w >>= 1) {
-      if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[q] = sh[0];
-    __syncthreads();
+  for (int q = 0; q < 16; ++q) {
+    float r = acc[q];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) r += __shfl_xor(r, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][q] = r;
+  }
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    float r = 0.f;
+#pragma unroll
+    for (int w = 0; w < kUT / 64; ++w) r += sh[w][threadIdx.x];
+    part[((size_t)c * 27 + tap) * 16 + threadIdx.x] = r;
   }
 }
 
@@ -507,25 +627,22 @@ __global__ void __launch_bounds__(kUT) k_pool_bwd(const bf16 *dY, bf16 *dX, int 
   dX[o] = f2bf(accumulate ? bf2f(dX[o]) + g : g);
 }
 
-// Y[v] = [ up(U)[v] (CU channels) , S[v] (CS channels) ] at the fine level
-__global__ void __launch_bounds__(kUT) k_upcat(const bf16 *U, int CU, const bf16 *S, int CS, bf16 *Y, int n0, int n1,
-                                              int n2, const int *done) {
+// Y[v] = [ up(U)[v] (CU channels) , S[v] (CS channels) ] at the fine level,
+// 8 channels (16 bytes) a thread: 45 us at 64^3 with a thread a channel, now 9
+__global__ void __launch_bounds__(kUT) k_upcat(const bf16 *__restrict__ U, int CU, const bf16 *__restrict__ S, int CS,
+                                              bf16 *__restrict__ Y, int n0, int n1, int n2, const int *done) {
   if (gated(done)) return;
-  const int C = CU + CS;
-  const size_t t = (size_t)blockIdx.x * kUT + threadIdx.x;
-  if (t >= (size_t)n0 * n1 * n2 * C) return;
-  const int c = (int)(t % C);
-  const int v = (int)(t / C);
+  const int C = CU + CS, C8 = C / 8;
+  const unsigned t = blockIdx.x * kUT + threadIdx.x;
+  if (t >= (unsigned)(n0 * n1 * n2) * C8) return;
+  const int c = (int)(t % C8) * 8;
+  const int v = (int)(t / C8);
   const int i = v % n0, j = (v / n0) % n1, k = v / (n0 * n1);
   const int pv = pvox(v, n0, n1);
-  bf16 val;
-  if (c < CU) {
-    const int N0 = n0 / 2, N1 = n1 / 2;
-    val = U[(size_t)(((k / 2 + 1) * (N1 + 2) + (j / 2 + 1)) * (N0 + 2) + (i / 2 + 1)) * CU + c];
-  } else {
-    val = S[(size_t)pv * CS + (c - CU)];
-  }
-  Y[(size_t)pv * C + c] = val;
+  const int N0 = n0 / 2, N1 = n1 / 2;
+  const bf16 *from = c < CU ? U + (size_t)(((k / 2 + 1) * (N1 + 2) + (j / 2 + 1)) * (N0 + 2) + (i / 2 + 1)) * CU + c
+                            : S + (size_t)pv * CS + (c - CU);
+  *reinterpret_cast<u16x8 *>(Y + (size_t)pv * C + c) = *reinterpret_cast<const u16x8 *>(from);
 }
 
 // upcat backward: dU[V][c] = sum of the 8 children's dY[child][c]; dS[v][c] = dY[v][CU + c]
@@ -612,6 +729,19 @@ __global__ void __launch_bounds__(kUT) k_pack32(const float *W, int Cin, int Cou
 }
 
 // BF16-rounded FP32 copy of the small layers' weights (the values the network uses)
+// first layer (k_conv_in): step s, lane: k = 32 s + 8 (lane / 16) ..+8 of the
+// 27 x 4 (tap, channel) pairs, zeros past them
+__global__ void __launch_bounds__(kUT) k_pack_in(const float *W, u16x8 *WB) {
+  const int lane = threadIdx.x & 63, s = threadIdx.x >> 6;
+  u16x8 r;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int k = 32 * s + (lane >> 4) * 8 + j;
+    r[j] = k < 108 ? f2bf(W[k * 16 + (lane & 15)]) : (bf16)0;
+  }
+  WB[threadIdx.x] = r;
+}
+
 __global__ void __launch_bounds__(kUT) k_round_bf16(const float *W, float *Wr, size_t n) {
   const size_t t = (size_t)blockIdx.x * kUT + threadIdx.x;
   if (t < n) Wr[t] = bf2f(f2bf(W[t]));
@@ -714,19 +844,23 @@ __global__ void __launch_bounds__(kUT) k_prec_input(const float *f0, const float
   for (int c = 0; c < 3; ++c) X[(size_t)pv * 4 + 1 + c] = f2bf(geom[c * np + pv]);
 }
 
-// bias gradient of the out layer: sum of dout over the interior
-__global__ void __launch_bounds__(kUT) k_sum_interior(const float *a, int n0, int n1, int n2, float *out, int accumulate) {
+// bias gradient of the out layer: part[block] = sum of dout over the block's
+// chunk of the interior; k_reduce_chunks adds the blocks (one block over all
+// voxels took 48 us at 32^3)
+__global__ void __launch_bounds__(kUT) k_sum_part(const float *__restrict__ a, int n0, int n1, int n2, int chunk,
+                                                 float *__restrict__ part) {
   __shared__ float sh[kUT];
   const int nvox = n0 * n1 * n2;
+  const int v0 = blockIdx.x * chunk, v1 = min(nvox, v0 + chunk);
   float s = 0.f;
-  for (int v = threadIdx.x; v < nvox; v += kUT) s += a[pvox(v, n0, n1)];
+  for (int v = v0 + threadIdx.x; v < v1; v += kUT) s += a[pvox(v, n0, n1)];
   sh[threadIdx.x] = s;
   __syncthreads();
   for (int w = kUT / 2; w > 0; w >>= 1) {
     if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = accumulate ? out[0] + sh[0] : sh[0];
+  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
 // ---- lane-layout self check of the MFMA fragments the kernels assume
@@ -784,13 +918,16 @@ struct moons_unet_s {
   size_t nparam = 0;
   float *W = nullptr, *G = nullptr, *Am = nullptr, *Av = nullptr, *Wr = nullptr; // master, grad, Adam m/v, rounded
   s16x4 *WB[11] = {}, *WT[11] = {};
-  u16x8 *WB32[11] = {}, *WT32[11] = {}; // k_conv_tile fragments (finest-level layers)
+  u16x8 *WB32[11] = {}, *WT32[11] = {}; // k_conv_tile fragments (levels 0 and 1)
+  u16x8 *WBin = nullptr;                // k_conv_in fragments
+  char *frag = nullptr;                 // the allocation that holds all of them
   int adam_t = 0;
   // activations for one grid size
   int n[3] = {0, 0, 0};
   Buf in, a0, e1, p1, a2, e2, p2, a4, b, c2, a6, d2, c1, a8, d1;
   Buf g_d1, g_a8, g_c1, g_d2, g_a6, g_c2, g_b, g_a4, g_p2, g_e2, g_a2, g_p1, g_e1, g_a0;
   float *out = nullptr, *dout = nullptr, *part = nullptr;
+  float *hin = nullptr, *htgt = nullptr; // device copies of the host entry points' input and target
   size_t part_n = 0;
   std::vector<void *> act_allocs;
 };
@@ -848,16 +985,29 @@ int ensure_acts(moons_unet_s *U, int n0, int n1, int n2) {
   U->part_n = std::max<size_t>((size_t)64 * 27 * 96 * 64, ublk((size_t)n0 * n1 * n2) + 16);
   if (hipMalloc(&U->part, U->part_n * sizeof(float)) != hipSuccess) return fail(MOONS_ERR_HIP, "unet: hipMalloc failed");
   U->act_allocs.push_back(U->part);
+  // kept with the activations: allocating and freeing them in each call of the
+  // host entry points took 0.1 ms and a device synchronisation
+  if (hipMalloc(&U->hin, 5 * np * sizeof(float)) != hipSuccess) return fail(MOONS_ERR_HIP, "unet: hipMalloc failed");
+  U->act_allocs.push_back(U->hin);
+  U->htgt = U->hin + 4 * np;
   return MOONS_OK;
 }
 
 // fragments of k_pack32 for a convolution of Ci input and Co output channels
 size_t pack32_n(int Ci, int Co) { return (size_t)((27 * (Ci / 16) + 1) / 2) * (Co / 16) * 64; }
 
-// the (Cin, Cout) pairs k_conv_tile is instantiated for
-bool tile_conv(int Ci, int Co) { return (Ci == 16 && Co == 16) || (Ci == 48 && Co == 16) || (Ci == 16 && Co == 48); }
+// the (Cin, Cout) pairs k_conv_tile is instantiated for: those of the finest
+// level, and of the next one (used there from kTileBlocks workgroups: 32 -> 32
+// at 32^3 14 us against 28 with a wave's own loads; the 96-channel layer's halo
+// and weights leave too few waves, 84 us against 36, and keep the tap split)
+bool tile_conv0(int Ci, int Co) { return (Ci == 16 && Co == 16) || (Ci == 48 && Co == 16) || (Ci == 16 && Co == 48); }
+bool tile_conv(int Ci, int Co) {
+  return tile_conv0(Ci, Co) || (Ci == 16 && Co == 32) || (Ci == 32 && (Co == 16 || Co == 32));
+}
+constexpr int kTileBlocks = 256;
 
 int pack_weights(moons_unet_s *U) {
+  hipLaunchKernelGGL(k_pack_in, dim3(1), dim3(kUT), 0, stream(), U->W + U->L[0].w_off, U->WBin);
   for (int l = 1; l <= 9; ++l) {
     const Layer &L = U->L[l];
     const size_t nf = (size_t)27 * (L.Cin / 16) * (L.Cout / 16) * 64;
@@ -892,22 +1042,24 @@ static void conv_split(const moons_unet_s *U, const s16x4 *WB, const float *bias
 void conv_mfma(const moons_unet_s *U, const s16x4 *WB, const float *bias, const Buf &X, Buf &Y, int n0, int n1, int n2,
                int relu, const int *done, const u16x8 *WB32 = nullptr) {
   const int nvox = n0 * n1 * n2;
-  if (WB32 && n0 % kCTX == 0 && n1 % kCTY == 0 && n2 % kCTZ == 0 && tile_conv(X.C, Y.C)) {
+  if (WB32 && n0 % kCTX == 0 && n1 % kCTY == 0 && n2 % kCTZ == 0 && tile_conv(X.C, Y.C) &&
+      (tile_conv0(X.C, Y.C) || nvox / (kCTX * kCTY * kCTZ) >= kTileBlocks)) {
     // tiles per workgroup along z: keep at least 2048 workgroups (8 a CU)
     const int tz = n2 / kCTZ, wxy = (n0 / kCTX) * (n1 / kCTY);
     int zt = 1;
     while (tz % (2 * zt) == 0 && (size_t)wxy * (tz / (2 * zt)) >= 2048) zt *= 2;
     const dim3 grid((unsigned)(n0 / kCTX), (unsigned)(n1 / kCTY), (unsigned)(tz / zt));
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream(), X.d, WB32, bias, Y.d, n0, n1, n2, relu, zt, done);
+    };
     if (X.C == 16 && Y.C == 16) {
       const int timer = bias ? MOONS_KTIMER_UNET_CONV16 : 0; // forward layers carry a bias
       ktimer_mark(timer);
-      hipLaunchKernelGGL((k_conv_tile<1, 1>), grid, dim3(256), 0, stream(), X.d, WB32, bias, Y.d, n0, n1, n2, relu, zt, done);
+      launch(k_conv_tile<1, 1>);
       ktimer_mark(timer);
-    }
-    else if (X.C == 48)
-      hipLaunchKernelGGL((k_conv_tile<3, 1>), grid, dim3(256), 0, stream(), X.d, WB32, bias, Y.d, n0, n1, n2, relu, zt, done);
-    else
-      hipLaunchKernelGGL((k_conv_tile<1, 3>), grid, dim3(256), 0, stream(), X.d, WB32, bias, Y.d, n0, n1, n2, relu, zt, done);
+    } else if (X.C == 48) launch(k_conv_tile<3, 1>);
+    else if (X.C == 16) Y.C == 32 ? launch(k_conv_tile<1, 2>) : launch(k_conv_tile<1, 3>);
+    else Y.C == 16 ? launch(k_conv_tile<2, 1>) : launch(k_conv_tile<2, 2>);
     return;
   }
   const unsigned grid = (unsigned)((nvox + 127) / 128);
@@ -947,43 +1099,72 @@ int forward(moons_unet_s *U, float *out, const float *scale, const int *done) {
   const int n0 = U->n[0], n1 = U->n[1], n2 = U->n[2];
   const float *W = U->Wr;
   auto nv = [&](int lev) { return (size_t)(n0 >> lev) * (n1 >> lev) * (n2 >> lev); };
-  hipLaunchKernelGGL(k_conv_in, dim3(ublk(16 * nv(0))), dim3(kUT), 0, stream(), U->in.d, W + U->L[0].w_off,
-                     U->W + U->L[0].b_off, U->a0.d, n0, n1, n2, done);
+  hipLaunchKernelGGL(k_conv_in, dim3((unsigned)((nv(0) + 64 * kInGroups - 1) / (64 * kInGroups))), dim3(kUT), 0, stream(),
+                     U->in.d, U->WBin, U->W + U->L[0].b_off, U->a0.d, n0, n1, n2, done);
   conv_mfma(U, U->WB[1], U->W + U->L[1].b_off, U->a0, U->e1, n0, n1, n2, 1, done, U->WB32[1]);
   hipLaunchKernelGGL(k_pool, dim3(ublk(nv(1) * 16)), dim3(kUT), 0, stream(), U->e1.d, U->p1.d, 16, n0 / 2, n1 / 2, n2 / 2, done);
-  conv_mfma(U, U->WB[2], U->W + U->L[2].b_off, U->p1, U->a2, n0 / 2, n1 / 2, n2 / 2, 1, done);
-  conv_mfma(U, U->WB[3], U->W + U->L[3].b_off, U->a2, U->e2, n0 / 2, n1 / 2, n2 / 2, 1, done);
+  conv_mfma(U, U->WB[2], U->W + U->L[2].b_off, U->p1, U->a2, n0 / 2, n1 / 2, n2 / 2, 1, done, U->WB32[2]);
+  conv_mfma(U, U->WB[3], U->W + U->L[3].b_off, U->a2, U->e2, n0 / 2, n1 / 2, n2 / 2, 1, done, U->WB32[3]);
   hipLaunchKernelGGL(k_pool, dim3(ublk(nv(2) * 32)), dim3(kUT), 0, stream(), U->e2.d, U->p2.d, 32, n0 / 4, n1 / 4, n2 / 4, done);
   conv_mfma(U, U->WB[4], U->W + U->L[4].b_off, U->p2, U->a4, n0 / 4, n1 / 4, n2 / 4, 1, done);
   conv_mfma(U, U->WB[5], U->W + U->L[5].b_off, U->a4, U->b, n0 / 4, n1 / 4, n2 / 4, 1, done);
-  hipLaunchKernelGGL(k_upcat, dim3(ublk(nv(1) * 96)), dim3(kUT), 0, stream(), U->b.d, 64, U->e2.d, 32, U->c2.d, n0 / 2, n1 / 2, n2 / 2, done);
-  conv_mfma(U, U->WB[6], U->W + U->L[6].b_off, U->c2, U->a6, n0 / 2, n1 / 2, n2 / 2, 1, done);
-  conv_mfma(U, U->WB[7], U->W + U->L[7].b_off, U->a6, U->d2, n0 / 2, n1 / 2, n2 / 2, 1, done);
-  hipLaunchKernelGGL(k_upcat, dim3(ublk(nv(0) * 48)), dim3(kUT), 0, stream(), U->d2.d, 32, U->e1.d, 16, U->c1.d, n0, n1, n2, done);
+  hipLaunchKernelGGL(k_upcat, dim3(ublk(nv(1) * 12)), dim3(kUT), 0, stream(), U->b.d, 64, U->e2.d, 32, U->c2.d, n0 / 2, n1 / 2, n2 / 2, done);
+  conv_mfma(U, U->WB[6], U->W + U->L[6].b_off, U->c2, U->a6, n0 / 2, n1 / 2, n2 / 2, 1, done, U->WB32[6]);
+  conv_mfma(U, U->WB[7], U->W + U->L[7].b_off, U->a6, U->d2, n0 / 2, n1 / 2, n2 / 2, 1, done, U->WB32[7]);
+  hipLaunchKernelGGL(k_upcat, dim3(ublk(nv(0) * 6)), dim3(kUT), 0, stream(), U->d2.d, 32, U->e1.d, 16, U->c1.d, n0, n1, n2, done);
   conv_mfma(U, U->WB[8], U->W + U->L[8].b_off, U->c1, U->a8, n0, n1, n2, 1, done, U->WB32[8]);
   conv_mfma(U, U->WB[9], U->W + U->L[9].b_off, U->a8, U->d1, n0, n1, n2, 1, done, U->WB32[9]);
-  hipLaunchKernelGGL(k_conv_out, dim3(ublk(16 * nv(0))), dim3(kUT), 0, stream(), U->d1.d, W + U->L[10].w_off,
+  hipLaunchKernelGGL(k_conv_out, dim3((unsigned)((n0 + kOX - 1) / kOX), (unsigned)((n1 + kOY - 1) / kOY), (unsigned)((n2 + kOZ - 1) / kOZ)),
+                     dim3(kUT), 0, stream(), U->d1.d, W + U->L[10].w_off,
                      U->W + U->L[10].b_off, out, n0, n1, n2, scale, done);
   MOONS_LAUNCH_CHECK();
   return MOONS_OK;
+}
+
+// Chunks of about `least` voxels or more, at most kMaxChunks: the partial-sum
+// kernels run a block a chunk (and tap), so that a coarse level still has
+// enough waves to hide their loads.  With 2048 voxels a chunk and a wave a tap
+// the weight gradients of the 16^3 level ran 54 waves, 127 us each, those of
+// 48 channels at 32^3 139 us; now 15 and 21.
+constexpr int kMaxChunks = 128;
+struct Chunks {
+  int n, size;
+};
+Chunks chunks_of(int nvox, int least, int step, int most = kMaxChunks) {
+  Chunks c;
+  c.n = std::max(1, std::min(most, nvox / least));
+  c.size = ((nvox + c.n - 1) / c.n + step - 1) / step * step;
+  c.n = (nvox + c.size - 1) / c.size;
+  return c;
+}
+
+// db of a layer (accumulated into G when acc)
+void grad_bias(moons_unet_s *U, const Layer &L, const bf16 *dY, int n0, int n1, int n2, int acc) {
+  const Chunks c = chunks_of(n0 * n1 * n2, 256, 1);
+  hipLaunchKernelGGL(k_dbias_part, dim3(c.n), dim3(kUT), 0, stream(), dY, L.Cout, n0, n1, n2, c.size, U->part);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(ublk(L.Cout)), dim3(kUT), 0, stream(), U->part, c.n, (size_t)L.Cout,
+                     U->G + L.b_off, acc);
 }
 
 // dW and db of an MFMA layer (accumulated into G when acc)
 void grad_mfma(moons_unet_s *U, int l, const Buf &X, const Buf &dY, int n0, int n1, int n2, int acc) {
   const Layer &L = U->L[l];
   const int nvox = n0 * n1 * n2;
-  int nchunk = std::max(1, std::min(64, nvox / 2048));
-  const int chunk = ((nvox + nchunk - 1) / nchunk + 15) / 16 * 16;
-  nchunk = (nvox + chunk - 1) / chunk;
-  const dim3 grid(nchunk, 27 * (L.Cin / 16));
-  switch (L.Cout / 16) {
-    case 1: hipLaunchKernelGGL(k_conv_dw<1>, grid, dim3(64), 0, stream(), X.d, L.Cin, dY.d, n0, n1, n2, chunk, U->part); break;
-    case 2: hipLaunchKernelGGL(k_conv_dw<2>, grid, dim3(64), 0, stream(), X.d, L.Cin, dY.d, n0, n1, n2, chunk, U->part); break;
-    default: hipLaunchKernelGGL(k_conv_dw<4>, grid, dim3(64), 0, stream(), X.d, L.Cin, dY.d, n0, n1, n2, chunk, U->part); break;
-  }
   const size_t nw = (size_t)27 * L.Cin * L.Cout;
+  const Chunks c = chunks_of(nvox, 128, 16, std::min<int>(kMaxChunks, (int)(U->part_n / nw)));
+  const int nchunk = c.n, chunk = c.size;
+  const dim3 grid(nchunk, 9 * (L.Cin / 16));
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(64), 0, stream(), X.d, L.Cin, dY.d, n0, n1, n2, chunk, U->part);
+  };
+  const bool rows = n0 % 4 == 0;
+  switch (L.Cout / 16) {
+    case 1: rows ? launch(k_conv_dw<1, true>) : launch(k_conv_dw<1, false>); break;
+    case 2: rows ? launch(k_conv_dw<2, true>) : launch(k_conv_dw<2, false>); break;
+    default: rows ? launch(k_conv_dw<4, true>) : launch(k_conv_dw<4, false>); break;
+  }
   hipLaunchKernelGGL(k_reduce_chunks, dim3(ublk(nw)), dim3(kUT), 0, stream(), U->part, nchunk, nw, U->G + L.w_off, acc);
-  hipLaunchKernelGGL(k_dbias, dim3(L.Cout), dim3(kUT), 0, stream(), dY.d, L.Cout, n0, n1, n2, U->G + L.b_off, acc);
+  grad_bias(U, L, dY.d, n0, n1, n2, acc);
 }
 
 // full backward pass from dout; parameter gradients into G (accumulated when acc)
@@ -996,11 +1177,9 @@ int backward(moons_unet_s *U, int acc) {
   {
     const Layer &L = U->L[10];
     const int nvox = (int)nv(0);
-    int nchunk = std::max(1, std::min(64, nvox / 4096));
-    const int chunk = (nvox + nchunk - 1) / nchunk;
-    nchunk = (nvox + chunk - 1) / chunk;
-    hipLaunchKernelGGL((k_small_dw<16, 1>), dim3(nchunk, 27), dim3(kUT), 0, stream(), U->d1.d, nullptr, U->dout, n0, n1,
-                       n2, chunk, U->part);
+    const Chunks c = chunks_of(nvox, 512, 1);
+    const int nchunk = c.n, chunk = c.size;
+    hipLaunchKernelGGL(k_out_dw, dim3(nchunk, 27), dim3(kUT), 0, stream(), U->d1.d, U->dout, n0, n1, n2, chunk, U->part);
     hipLaunchKernelGGL(k_reduce_chunks, dim3(ublk(27 * 16)), dim3(kUT), 0, stream(), U->part, nchunk, (size_t)27 * 16,
                        U->G + L.w_off, acc);
     hipLaunchKernelGGL(k_conv_out_dx, dim3(ublk(nv(0))), dim3(kUT), 0, stream(), U->dout, Wr + L.w_off, U->g_d1.d, n0, n1, n2);
@@ -1050,14 +1229,12 @@ int backward(moons_unet_s *U, int acc) {
   {
     const Layer &L = U->L[0];
     const int nvox = (int)nv(0);
-    int nchunk = std::max(1, std::min(64, nvox / 4096));
-    const int chunk = (nvox + nchunk - 1) / nchunk;
-    nchunk = (nvox + chunk - 1) / chunk;
-    hipLaunchKernelGGL((k_small_dw<4, 16>), dim3(nchunk, 27), dim3(kUT), 0, stream(), U->in.d, U->g_a0.d, nullptr, n0,
-                       n1, n2, chunk, U->part);
+    const Chunks c = chunks_of(nvox, 256, 16);
+    const int nchunk = c.n, chunk = c.size;
+    hipLaunchKernelGGL(k_conv_dw_in, dim3(nchunk, 9), dim3(64), 0, stream(), U->in.d, U->g_a0.d, n0, n1, n2, chunk, U->part);
     hipLaunchKernelGGL(k_reduce_chunks, dim3(ublk(27 * 64)), dim3(kUT), 0, stream(), U->part, nchunk, (size_t)27 * 64,
                        U->G + L.w_off, acc);
-    hipLaunchKernelGGL(k_dbias, dim3(16), dim3(kUT), 0, stream(), U->g_a0.d, 16, n0, n1, n2, U->G + L.b_off, acc);
+    grad_bias(U, L, U->g_a0.d, n0, n1, n2, acc);
   }
   MOONS_LAUNCH_CHECK();
   return MOONS_OK;
@@ -1066,8 +1243,10 @@ int backward(moons_unet_s *U, int acc) {
 int backward_all(moons_unet_s *U, int acc) {
   int st = backward(U, acc);
   if (st) return st;
-  hipLaunchKernelGGL(k_sum_interior, dim3(1), dim3(kUT), 0, stream(), U->dout, U->n[0], U->n[1], U->n[2],
-                     U->G + U->L[10].b_off, acc);
+  const Chunks c = chunks_of(U->n[0] * U->n[1] * U->n[2], 512, 1);
+  hipLaunchKernelGGL(k_sum_part, dim3(c.n), dim3(kUT), 0, stream(), U->dout, U->n[0], U->n[1], U->n[2], c.size, U->part);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(1), dim3(kUT), 0, stream(), U->part, c.n, (size_t)1, U->G + U->L[10].b_off,
+                     acc);
   MOONS_LAUNCH_CHECK();
   return MOONS_OK;
 }
@@ -1176,6 +1355,18 @@ void unet_prec_destroy(UnetPrec *P) {
 
 extern "C" {
 
+// He initialisation (normal, std sqrt(2 / fan_in)), biases zero
+static std::vector<float> he_weights(const moons_unet_s *U, unsigned long long seed) {
+  std::vector<float> w(U->nparam, 0.f);
+  std::mt19937_64 rng(seed);
+  for (int l = 0; l < 11; ++l) {
+    const float sd = std::sqrt(2.f / (27.f * U->L[l].Cin)) * (l == 10 ? 0.5f : 1.f);
+    std::normal_distribution<float> nd(0.f, sd);
+    for (size_t q = 0; q < (size_t)27 * U->L[l].Cin * U->L[l].Cout; ++q) w[U->L[l].w_off + q] = nd(rng);
+  }
+  return w;
+}
+
 int moons_unet_create(unsigned long long seed, moons_unet_t *out) {
   if (!stream()) return fail(MOONS_ERR_STATE, "moons_init has not been called");
   if (!out) return fail(MOONS_ERR_ARG, "moons_unet_create: null argument");
@@ -1191,23 +1382,35 @@ int moons_unet_create(unsigned long long seed, moons_unet_t *out) {
     off += U->L[l].Cout;
   }
   U->nparam = off;
-  // He initialisation (normal, std sqrt(2 / fan_in)), biases zero
-  std::vector<float> w(off, 0.f);
-  std::mt19937_64 rng(seed);
-  for (int l = 0; l < 11; ++l) {
-    const float sd = std::sqrt(2.f / (27.f * U->L[l].Cin)) * (l == 10 ? 0.5f : 1.f);
-    std::normal_distribution<float> nd(0.f, sd);
-    for (size_t q = 0; q < (size_t)27 * U->L[l].Cin * U->L[l].Cout; ++q) w[U->L[l].w_off + q] = nd(rng);
-  }
+  const std::vector<float> w = he_weights(U, seed);
   bool ok = hipMalloc(&U->W, off * 4) == hipSuccess && hipMalloc(&U->G, off * 4) == hipSuccess &&
             hipMalloc(&U->Am, off * 4) == hipSuccess && hipMalloc(&U->Av, off * 4) == hipSuccess &&
             hipMalloc(&U->Wr, off * 4) == hipSuccess;
-  for (int l = 1; l <= 9 && ok; ++l) {
-    const size_t nf = (size_t)27 * (U->L[l].Cin / 16) * (U->L[l].Cout / 16) * 64;
-    ok = hipMalloc(&U->WB[l], nf * sizeof(s16x4)) == hipSuccess && hipMalloc(&U->WT[l], nf * sizeof(s16x4)) == hipSuccess;
-    if (ok && U->L[l].lev == 0 && tile_conv(U->L[l].Cin, U->L[l].Cout))
-      ok = hipMalloc(&U->WB32[l], pack32_n(U->L[l].Cin, U->L[l].Cout) * sizeof(u16x8)) == hipSuccess &&
-           hipMalloc(&U->WT32[l], pack32_n(U->L[l].Cout, U->L[l].Cin) * sizeof(u16x8)) == hipSuccess;
+  // every layer's weight fragments in one allocation, each block 16-byte aligned
+  auto place = [&](bool assign) {
+    size_t at = kUT * sizeof(u16x8);
+    auto take = [&](size_t bytes) {
+      char *q = assign ? U->frag + at : nullptr;
+      at += (bytes + 15) / 16 * 16;
+      return q;
+    };
+    for (int l = 1; l <= 9; ++l) {
+      const Layer &L = U->L[l];
+      const size_t nf = (size_t)27 * (L.Cin / 16) * (L.Cout / 16) * 64 * sizeof(s16x4);
+      U->WB[l] = reinterpret_cast<s16x4 *>(take(nf));
+      U->WT[l] = reinterpret_cast<s16x4 *>(take(nf));
+      if (L.lev <= 1 && tile_conv(L.Cin, L.Cout)) {
+        U->WB32[l] = reinterpret_cast<u16x8 *>(take(pack32_n(L.Cin, L.Cout) * sizeof(u16x8)));
+        U->WT32[l] = reinterpret_cast<u16x8 *>(take(pack32_n(L.Cout, L.Cin) * sizeof(u16x8)));
+      }
+    }
+    return at;
+  };
+  const size_t frag = place(false);
+  ok = ok && hipMalloc(&U->frag, frag) == hipSuccess;
+  if (ok) {
+    U->WBin = reinterpret_cast<u16x8 *>(U->frag);
+    place(true);
   }
   if (!ok) {
     moons_unet_destroy(U);
@@ -1233,12 +1436,7 @@ int moons_unet_destroy(moons_unet_t U) {
   free_acts(U);
   for (float *p : {U->W, U->G, U->Am, U->Av, U->Wr})
     if (p) (void)hipFree(p);
-  for (int l = 0; l < 11; ++l) {
-    if (U->WB[l]) (void)hipFree(U->WB[l]);
-    if (U->WT[l]) (void)hipFree(U->WT[l]);
-    if (U->WB32[l]) (void)hipFree(U->WB32[l]);
-    if (U->WT32[l]) (void)hipFree(U->WT32[l]);
-  }
+  if (U->frag) (void)hipFree(U->frag);
   delete U;
   return MOONS_OK;
 }
@@ -1267,16 +1465,13 @@ int moons_unet_forward_host(moons_unet_t U, int n0, int n1, int n2, const float 
   int st = ensure_acts(U, n0, n1, n2);
   if (st) return st;
   const size_t np = padded(U, 0);
-  float *d = nullptr;
-  MOONS_HIP(hipMalloc(&d, 4 * np * sizeof(float)));
-  MOONS_HIP(hipMemcpyAsync(d, in4, 4 * np * sizeof(float), hipMemcpyHostToDevice, stream()));
-  hipLaunchKernelGGL(k_input, dim3(ublk((size_t)n0 * n1 * n2)), dim3(kUT), 0, stream(), d, U->in.d, n0, n1, n2);
+  MOONS_HIP(hipMemcpyAsync(U->hin, in4, 4 * np * sizeof(float), hipMemcpyHostToDevice, stream()));
+  hipLaunchKernelGGL(k_input, dim3(ublk((size_t)n0 * n1 * n2)), dim3(kUT), 0, stream(), U->hin, U->in.d, n0, n1, n2);
   st = forward(U, U->out, nullptr, nullptr);
   if (!st) {
     MOONS_HIP(hipMemcpyAsync(out, U->out, np * sizeof(float), hipMemcpyDeviceToHost, stream()));
     MOONS_HIP(hipStreamSynchronize(stream()));
   }
-  (void)hipFree(d);
   return st;
 }
 
@@ -1287,18 +1482,13 @@ int moons_unet_grad_host(moons_unet_t U, int n0, int n1, int n2, const float *in
   int st = ensure_acts(U, n0, n1, n2);
   if (st) return st;
   const size_t np = padded(U, 0);
-  float *d = nullptr, *t = nullptr;
-  MOONS_HIP(hipMalloc(&d, 4 * np * sizeof(float)));
-  MOONS_HIP(hipMalloc(&t, np * sizeof(float)));
-  MOONS_HIP(hipMemcpyAsync(d, in4, 4 * np * sizeof(float), hipMemcpyHostToDevice, stream()));
-  MOONS_HIP(hipMemcpyAsync(t, target, np * sizeof(float), hipMemcpyHostToDevice, stream()));
-  hipLaunchKernelGGL(k_input, dim3(ublk((size_t)n0 * n1 * n2)), dim3(kUT), 0, stream(), d, U->in.d, n0, n1, n2);
-  if (!(st = forward(U, U->out, nullptr, nullptr)) && !(st = loss(U, t, l)) && !(st = backward_all(U, 0))) {
+  MOONS_HIP(hipMemcpyAsync(U->hin, in4, 4 * np * sizeof(float), hipMemcpyHostToDevice, stream()));
+  MOONS_HIP(hipMemcpyAsync(U->htgt, target, np * sizeof(float), hipMemcpyHostToDevice, stream()));
+  hipLaunchKernelGGL(k_input, dim3(ublk((size_t)n0 * n1 * n2)), dim3(kUT), 0, stream(), U->hin, U->in.d, n0, n1, n2);
+  if (!(st = forward(U, U->out, nullptr, nullptr)) && !(st = loss(U, U->htgt, l)) && !(st = backward_all(U, 0))) {
     MOONS_HIP(hipMemcpyAsync(grad, U->G, U->nparam * 4, hipMemcpyDeviceToHost, stream()));
     MOONS_HIP(hipStreamSynchronize(stream()));
   }
-  (void)hipFree(d);
-  (void)hipFree(t);
   return st;
 }
 
