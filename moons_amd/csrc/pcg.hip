@@ -9,8 +9,9 @@
 // modify_RHS_SF (code/handwritten/solvers/PCG/PCG_aux.f90:30-54).
 //
 // A Jacobi solve of a grid that fits the CUs' registers and LDS (up to 128^3)
-// runs its whole loop as one resident kernel (pcg_resident.hpp).  Otherwise, in
-// a captured graph, and in the flexible PCG around the multigrid or the
+// runs its whole loop as one resident kernel (pcg_resident.hpp; in a captured
+// graph as three kernels an iteration over the same blocks, with the same
+// bits).  Otherwise, and in the flexible PCG around the multigrid or the
 // network, one iteration is three HBM-bound kernels over the interior cells:
 //   k_pcg_matvec   q = vol*lap(p), partial (p,q)              read p, write q        16 B/cell
 //   k_pcg_update   x += a p, r -= a q, partials (r,r),(Minv r,r) read x,p,r,q write x,r 48 B/cell
@@ -622,6 +623,7 @@ struct moons_pcg_s {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   ResPlan res;                  // the resident loop's box (cpt 0: the launch-per-kernel loop)
   unsigned long long *slots = nullptr;
+  double *part63 = nullptr;     // the boxes' block sums (3 a box), beside the slots
   int spins = 0;                // its waits' bound
   bool noalloc = false;         // a one-shot solver over the static scratch (no host_init)
 };
@@ -825,6 +827,25 @@ static int pcg_launch_iteration_mg(moons_pcg_s *S, double *x, int it) {
 
 static int pcg_launch_iteration(moons_pcg_s *S, double *x, int it) { return pcg_launch(S, x, it, 7); }
 
+// One Jacobi iteration over the resident loop's boxes (captured graphs).
+static int pcg_launch_iteration_boxes(moons_pcg_s *S, double *x, int it) {
+  const ResPlan &P = S->res;
+  const dim3 grid(P.nb()), block(kResNT);
+  double *part1 = S->part63, *part2 = S->part63 + P.nb();
+  if (S->op == MOONS_OP_NRG_DIFFUSION)
+    hipLaunchKernelGGL((k_box_matvec<kResNT, true>), grid, block, 0, stream(), S->p, S->q, S->G, P.by, P.gy, P.cpt, S->ctrl,
+                       part1, nrg_k(S));
+  else
+    hipLaunchKernelGGL((k_box_matvec<kResNT, false>), grid, block, 0, stream(), S->p, S->q, S->G, P.by, P.gy, P.cpt, S->ctrl,
+                       part1, nrg_k(S));
+  hipLaunchKernelGGL(k_box_update<kResNT>, grid, block, 0, stream(), x, S->p, S->r, S->q, S->G, P.by, P.gy, P.cpt, S->ctrl,
+                     part1, part2, it);
+  hipLaunchKernelGGL(k_box_pupdate<kResNT>, grid, block, 0, stream(), S->p, S->r, S->G, P.by, P.gy, P.cpt, S->ctrl, part2,
+                     it);
+  MOONS_LAUNCH_CHECK();
+  return MOONS_OK;
+}
+
 extern "C" {
 
 int moons_pcg_sf_create(moons_mesh_t m, int op, int prec, moons_field_t x, moons_pcg_t *out) {
@@ -872,10 +893,11 @@ int moons_pcg_sf_create(moons_mesh_t m, int op, int prec, moons_field_t x, moons
   }
   if (prec != MOONS_PREC_MG_FP32) {
     resident_setup(S);
-    if (S->res.cpt && hipMalloc(&S->slots, kResSlotWords * sizeof(unsigned long long)) != hipSuccess) {
+    if (S->res.cpt && hipMalloc(&S->slots, (kResSlotWords + 3 * kResMaxBlocks) * sizeof(double)) != hipSuccess) {
       moons_pcg_destroy(S);
       return fail(MOONS_ERR_HIP, "moons_pcg_sf_create: allocation failed");
     }
+    S->part63 = reinterpret_cast<double *>(S->slots) + kResSlotWords;
   }
   std::memset(S->host_init, 0xff, sizeof(PcgCtrl)); // differs from any real block: first upload writes it
   (void)hipMemsetAsync(S->r, 0, bytes, stream());
@@ -1068,7 +1090,8 @@ static int pcg_solve_impl(moons_pcg_s *S, moons_field_t x, moons_field_t b) {
   if (sync_free()) {
     // exactly iter_max iterations, gated on the device; nothing read back
     for (int it = 1; it <= S->iter_max; ++it) {
-      st = mg ? pcg_launch_iteration_mg(S, x->d, it) : pcg_launch_iteration(S, x->d, it);
+      st = mg ? pcg_launch_iteration_mg(S, x->d, it)
+              : S->res.cpt ? pcg_launch_iteration_boxes(S, x->d, it) : pcg_launch_iteration(S, x->d, it);
       if (st) return st;
     }
     return launch_apply_bcs(x, false);

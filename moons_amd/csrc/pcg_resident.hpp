@@ -35,7 +35,8 @@
 //
 // Residency: the grid never exceeds the number of CUs, one block a CU, and it
 // runs on the library's one stream only (never in a captured graph, whose
-// replays may share the GPU with each other).  Should blocks nevertheless not
+// replays may share the GPU with each other: there the kernels at the end of
+// this file do the same sums a launch at a time).  Should blocks nevertheless not
 // all be resident, every wait is bounded: a block that gives up sets `abort`,
 // the others see it while they wait, every block returns, x is untouched (the
 // result goes to a buffer that k_pcg_take copies only from a complete run),
@@ -92,6 +93,35 @@ struct ResShared {
   int bad;
 };
 
+// The block's sums of v[0..V) (as left in sh.part by every wave), for thread t < V.
+template <int NT>
+__device__ __forceinline__ double block_total(const ResShared<NT> &sh, int q) {
+  double s = 0.0;
+#pragma unroll
+  for (int u = 0; u < NT / kWave; ++u) s += sh.part[q][u];
+  return s;
+}
+template <int NT, int V>
+__device__ __forceinline__ void wave_totals(double (&v)[V], double (&to)[2][NT / kWave]) {
+#pragma unroll
+  for (int q = 0; q < V; ++q) v[q] = wave_sum63(v[q]);
+  if ((threadIdx.x & (kWave - 1)) == kWave - 1) {
+#pragma unroll
+    for (int q = 0; q < V; ++q) to[q][threadIdx.x / kWave] = v[q];
+  }
+}
+// The sums over nb blocks' values from the waves' sums in sh.all.
+template <int NT, int V>
+__device__ __forceinline__ void grid_totals(double (&v)[V], const ResShared<NT> &sh, int nb) {
+  const int nw = (nb + kWave - 1) / kWave;
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    double s = 0.0;
+    for (int u = 0; u < nw; ++u) s += sh.all[q][u];
+    v[q] = s;
+  }
+}
+
 // Sums v[0..V) over all blocks (slot set S of V x nb words); false when the
 // wait was given up, the same in every thread.  Stores issued before the call
 // have completed when the block's slot is published.
@@ -99,18 +129,11 @@ template <int NT, int V>
 __device__ __forceinline__ bool all_reduce(double (&v)[V], unsigned long long *S, int nb, ResShared<NT> &sh,
                                            unsigned long long *abort_, int spins) {
   const int t = threadIdx.x, w = t / kWave;
-#pragma unroll
-  for (int q = 0; q < V; ++q) v[q] = wave_sum63(v[q]);
-  if ((t & (kWave - 1)) == kWave - 1) {
-#pragma unroll
-    for (int q = 0; q < V; ++q) sh.part[q][w] = v[q];
-  }
+  wave_totals<NT, V>(v, sh.part);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (t < V) {
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < NT / kWave; ++u) s += sh.part[t][u];
+    const double s = block_total<NT>(sh, t);
     unsigned long long bits = (unsigned long long)__double_as_longlong(s);
     if (s != s) bits = 0x7ff8000000000000ull;
     agent_store(S + (size_t)t * nb + blockIdx.x, bits);
@@ -136,25 +159,14 @@ __device__ __forceinline__ bool all_reduce(double (&v)[V], unsigned long long *S
 #pragma unroll
       for (int q = 0; q < V; ++q) a[q] = __longlong_as_double((long long)b[q]);
     }
-#pragma unroll
-    for (int q = 0; q < V; ++q) a[q] = wave_sum63(a[q]);
-    if ((t & (kWave - 1)) == kWave - 1) {
-#pragma unroll
-      for (int q = 0; q < V; ++q) sh.all[q][w] = a[q];
-    }
+    wave_totals<NT, V>(a, sh.all);
   }
   __syncthreads();
   if (sh.bad) {
     if (t == 0) agent_store(abort_, 1ull);
     return false;
   }
-  const int nw = (nb + kWave - 1) / kWave;
-#pragma unroll
-  for (int q = 0; q < V; ++q) {
-    double s = 0.0;
-    for (int u = 0; u < nw; ++u) s += sh.all[q][u];
-    v[q] = s;
-  }
+  grid_totals<NT, V>(v, sh, nb);
   return true;
 }
 
@@ -484,6 +496,132 @@ __global__ void __launch_bounds__(NT) k_pcg_resident(const double *__restrict__ 
     ctrl->beta = beta;
     ctrl->rho[it & 1] = rho;
     ctrl->done = kResDone;
+  }
+}
+
+// ---- the same loop a kernel at a time, for a captured graph: the resident
+// loop's boxes, arithmetic and orders of summation, so that a replay equals
+// the eager solve bit for bit.  p's face ghosts are kept in memory here.
+struct Box {
+  int i, j, k0, nk; // the thread's column; nk 0: none
+};
+__device__ __forceinline__ Box box_of(const CCGeom &G, int by, int gy, int cpt) {
+  const int L = xcd_remap(blockIdx.x, gridDim.x), t = threadIdx.x, jj = t / G.n0, j0 = 1 + (L % gy) * by;
+  Box b;
+  b.i = 1 + t - jj * G.n0;
+  b.j = j0 + jj;
+  b.k0 = 1 + (L / gy) * cpt;
+  b.nk = jj < min(by, G.n1 + 1 - j0) ? min(cpt, G.n2 + 1 - b.k0) : 0;
+  return b;
+}
+// sums of the last kernel's V x nb block sums, the same in every block
+template <int NT, int V>
+__device__ __forceinline__ void box_sums(double (&v)[V], const double *part, int nb, ResShared<NT> &sh) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < V; ++q) v[q] = t < nb ? part[(size_t)q * nb + t] : 0.0;
+  wave_totals<NT, V>(v, sh.all);
+  __syncthreads();
+  grid_totals<NT, V>(v, sh, nb);
+}
+template <int NT, int V>
+__device__ __forceinline__ void box_put(double (&v)[V], double *part, int nb, ResShared<NT> &sh) {
+  wave_totals<NT, V>(v, sh.part);
+  __syncthreads();
+  if (threadIdx.x < V) part[(size_t)threadIdx.x * nb + blockIdx.x] = block_total<NT>(sh, threadIdx.x);
+}
+
+template <int NT, bool NRG>
+__global__ void __launch_bounds__(NT) k_box_matvec(const double *__restrict__ p, double *__restrict__ q, CCGeom G, int by,
+                                                  int gy, int cpt, const PcgCtrl *ctrl, double *part, NrgK K) {
+  if (ctrl->done) return;
+  __shared__ ResShared<NT> sh;
+  const Box b = box_of(G, by, gy, cpt);
+  const size_t sx = G.s0, sxy = (size_t)G.s0 * G.s1;
+  double acc[1] = {0.0};
+  if (b.nk > 0) {
+    const double dxy = G.c[0].dh[b.i] * G.c[1].dh[b.j];
+    const St6<double> SX = st6(G.c[0], b.i), SY = st6(G.c[1], b.j);
+#pragma unroll 4
+    for (int u = 0; u < b.nk; ++u) {
+      const int k = b.k0 + u;
+      const size_t o = (size_t)b.i + (size_t)b.j * sx + (size_t)k * sxy;
+      const double c = p[o];
+      const double v = NRG ? nrg7(K, G, c, p[o - 1], p[o + 1], p[o - sx], p[o + sx], p[o - sxy], p[o + sxy], b.i, b.j, k)
+                           : lap7s(c, p[o - 1], p[o + 1], p[o - sx], p[o + sx], p[o - sxy], p[o + sxy], SX, SY,
+                                   st6(G.c[2], k));
+      const double qv = v * (dxy * G.c[2].dh[k]);
+      q[o] = qv;
+      acc[0] += c * qv;
+    }
+  }
+  box_put<NT, 1>(acc, part, gridDim.x, sh);
+}
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_box_update(double *__restrict__ x, const double *__restrict__ p,
+                                                  double *__restrict__ r, const double *__restrict__ q, CCGeom G, int by,
+                                                  int gy, int cpt, PcgCtrl *ctrl, const double *part1, double *part2,
+                                                  int it) {
+  if (ctrl->done) return;
+  __shared__ ResShared<NT> sh;
+  const Box b = box_of(G, by, gy, cpt);
+  double pq[1];
+  box_sums<NT, 1>(pq, part1, gridDim.x, sh);
+  const double alpha = ctrl->rho[(it - 1) & 1] / pq[0], malpha = -alpha;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ctrl->pq = pq[0];
+    ctrl->alpha = alpha;
+  }
+  double two[2] = {0.0, 0.0};
+  if (b.nk > 0) {
+    const size_t sx = G.s0, sxy = (size_t)G.s0 * G.s1;
+    const double dxy = G.c[0].dh[b.i] * G.c[1].dh[b.j];
+    const double axy = G.c[0].lA[b.i] + G.c[0].lB[b.i] + G.c[1].lA[b.j] + G.c[1].lB[b.j];
+#pragma unroll 4
+    for (int u = 0; u < b.nk; ++u) {
+      const size_t o = (size_t)b.i + (size_t)b.j * sx + (size_t)(b.k0 + u) * sxy;
+      x[o] = x[o] + p[o] * alpha;
+      const double rn = r[o] + q[o] * malpha;
+      r[o] = rn;
+      two[0] += rn * rn;
+      const double z = minv_at<double>(G, dxy, axy, b.k0 + u) * rn;
+      two[1] += z * rn;
+    }
+  }
+  box_put<NT, 2>(two, part2, gridDim.x, sh);
+}
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_box_pupdate(double *__restrict__ p, const double *__restrict__ r, CCGeom G,
+                                                   int by, int gy, int cpt, PcgCtrl *ctrl, const double *part2, int it) {
+  if (ctrl->done) return;
+  __shared__ ResShared<NT> sh;
+  const Box b = box_of(G, by, gy, cpt);
+  double two[2];
+  box_sums<NT, 2>(two, part2, gridDim.x, sh);
+  const double rr = two[0], rz = two[1];
+  const ExitDecision e = exit_decision(ctrl, it, rr);
+  const double beta = rz / ctrl->rho[(it - 1) & 1];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    publish_exit(ctrl, it, rr, e);
+    ctrl->rz = rz;
+    ctrl->beta = beta;
+    ctrl->rho[it & 1] = rz;
+  }
+  if (e.stop || b.nk == 0) return;
+  const size_t sx = G.s0, sxy = (size_t)G.s0 * G.s1;
+  const double dxy = G.c[0].dh[b.i] * G.c[1].dh[b.j];
+  const double axy = G.c[0].lA[b.i] + G.c[0].lB[b.i] + G.c[1].lA[b.j] + G.c[1].lB[b.j];
+  const bool edge_ij = b.i == 1 || b.i == G.n0 || b.j == 1 || b.j == G.n1;
+#pragma unroll 4
+  for (int u = 0; u < b.nk; ++u) {
+    const int k = b.k0 + u;
+    const size_t o = (size_t)b.i + (size_t)b.j * sx + (size_t)k * sxy;
+    const double z = minv_at<double>(G, dxy, axy, k) * r[o];
+    const double pn = p[o] * beta + z;
+    p[o] = pn;
+    if (edge_ij || k == 1 || k == G.n2) fill_ghosts_implicit(p, G, b.i, b.j, k, pn);
   }
 }
 
