@@ -204,4 +204,39 @@ int launch_plane_scale(moons_field_s *u, int d, int idx, double val);
 int launch_cross(moons_field_s *out, const moons_field_s *a, const moons_field_s *b, const moons_field_s *c,
                  const moons_field_s *d, int sign);
 int launch_sub(moons_field_s *out, const moons_field_s *a, const moons_field_s *b);
+
+// ---- fused source terms (sources.hip).  A *_fits rule tells whether the fused
+// launch covers the call: locations and meshes as the kernel assumes, no
+// operand that is also a result, no gate.  What it does not cover runs as the
+// sequence of passes, which also refuses what cannot be computed.
+bool edges_fit(moons_field_s *const E[3], moons_field_s *const U_E[6], moons_field_s *const B[3],
+               moons_field_s *const tmp[6]);
+// E = U_E x face2Edge(B); tmp (optional): the six interpolants
+int launch_edge_cross(moons_field_s *const E[3], moons_field_s *const U_E[6], moons_field_s *const B[3],
+                      moons_field_s *const tmp[6]);
+int launch_face2edge(moons_field_s *const UE[6], moons_field_s *const U[3]); // face2Edge_no_diag
+bool curl3_fits(moons_field_s *const out[3], moons_field_s *const in[3]);
+int launch_curl3(moons_field_s *const out[3], moons_field_s *const in[3], bool scaled, double scale);
+// FB, the AB2 right-hand side of B* and B* = B, of the induction equation
+int launch_ind_source(moons_field_s *const E[3], moons_field_s *const J[3], moons_field_s *const sig[3],
+                      moons_field_s *const FB[3], moons_field_s *const B[3], moons_field_s *const rhs[3],
+                      moons_field_s *const Bstar[3], const int wall[3], double dt);
+int launch_btot(moons_field_s *const out[3], moons_field_s *const B0[3], moons_field_s *const B[3]);
+int launch_jxb(moons_field_s *const out[3], moons_field_s *const J[3], moons_field_s *const Bt[3], double N);
+bool div_fits(const moons_field_s *divU, moons_field_s *const u[3]);
+int launch_div(moons_field_s *divU, moons_field_s *const u[3], bool scaled, double scale);
+bool project_fits(moons_field_s *const X[3], moons_field_s *const Xstar[3], moons_field_s *const g[3],
+                  const moons_field_s *phi);
+int launch_project(moons_field_s *const X[3], moons_field_s *const Xstar[3], moons_field_s *const g[3],
+                   const moons_field_s *phi, double inv);
+// The momentum sources, the AB2 right-hand side and (Ustar not null) U* = U.
+struct MomSource {
+  moons_field_s *const *U, *const *UE, *const *F, *const *Fnm1, *const *rhs, *const *Ustar;
+  moons_field_s *const *jx;       // J x B on the fluid faces (may be rhs), or null
+  const moons_field_s *T;         // buoyancy's temperature, or null
+  const moons_field_s *const *g;  // gravity (buoyancy, gravity source)
+  int grav, wall[3];
+  double ce, dt, buoy_scale, grav_scale;
+};
+int launch_mom_source(const MomSource &S);
 }

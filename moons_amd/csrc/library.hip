@@ -1078,6 +1078,8 @@ int moons_div(moons_field_t divU, moons_field_t u, moons_field_t v, moons_field_
   if (!divU || !u || !v || !w) return fail(MOONS_ERR_ARG, "moons_div: null argument");
   if (u->dl != (divU->dl ^ 1) || v->dl != (divU->dl ^ 2) || w->dl != (divU->dl ^ 4))
     return fail(MOONS_ERR_ARG, "moons_div: component locations do not match the output");
+  moons_field_s *const uvw[3] = {u, v, w};
+  if (div_fits(divU, uvw)) return launch_div(divU, uvw, false, 1.0);
   int st;
   if ((st = launch_del(divU, u, 1, 0, 0, 1))) return st;
   if ((st = launch_del(divU, v, 1, 1, 0, 2))) return st;
@@ -1124,6 +1126,7 @@ int moons_edge_cross_face_E(moons_field_t E[3], moons_field_t U_E[6], moons_fiel
   }
   for (int d = 0; d < 3; ++d)
     if (E[d]->dl != edge_dl[d]) return fail(MOONS_ERR_ARG, "moons_edge_cross_face_E: E must be on edges");
+  if (edges_fit(E, U_E, B, tmp)) return launch_edge_cross(E, U_E, B, tmp);
   int st;
   for (int q = 0; q < 6; ++q) {
     const int orth = 3 - tmp_face[q] - tmp_edge[q];
@@ -1140,6 +1143,7 @@ int moons_advect_B(moons_field_t adv[3], moons_field_t U_E[6], moons_field_t B[3
                    moons_field_t temp_E[3]) {
   int st = moons_edge_cross_face_E(temp_E, U_E, B, temp_E_TF);
   if (st) return st;
+  if (adv && adv[0] && adv[1] && adv[2] && curl3_fits(adv, temp_E)) return launch_curl3(adv, temp_E, false, 1.0);
   for (int d = 0; d < 3; ++d)
     if ((st = moons_curl(adv[d], temp_E[0], temp_E[1], temp_E[2], d))) return st;
   return MOONS_OK;

@@ -1227,11 +1227,19 @@ int moons_clean_div(moons_pcg_t S, moons_field_t X[3], moons_field_t Xstar[3], m
   for (int d = 0; d < 3; ++d)
     if (!X[d] || !Xstar[d] || !temp_F[d]) return fail(MOONS_ERR_ARG, "moons_clean_div: null component");
   int st;
-  if ((st = moons_div(temp_CC, Xstar[0], Xstar[1], Xstar[2]))) return st;
-  if ((st = launch_scale(temp_CC, scale))) return st;
+  if (div_fits(temp_CC, Xstar)) {
+    if ((st = launch_div(temp_CC, Xstar, true, scale))) return st;
+  } else {
+    if ((st = moons_div(temp_CC, Xstar[0], Xstar[1], Xstar[2]))) return st;
+    if ((st = launch_scale(temp_CC, scale))) return st;
+  }
   if ((st = moons_pcg_sf_solve(S, phi, temp_CC, info))) return st;
-  if ((st = moons_grad(temp_F[0], temp_F[1], temp_F[2], phi))) return st;
   const double inv = 1.0 / scale;
+  if (project_fits(X, Xstar, temp_F, phi)) {
+    if ((st = launch_project(X, Xstar, temp_F, phi, inv))) return st;
+    return launch_apply_bcs3(X, false);
+  }
+  if ((st = moons_grad(temp_F[0], temp_F[1], temp_F[2], phi))) return st;
   for (int d = 0; d < 3; ++d) {
     if ((st = launch_scale(temp_F[d], inv))) return st;
     if ((st = launch_sub(X[d], Xstar[d], temp_F[d]))) return st;

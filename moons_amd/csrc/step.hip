@@ -50,15 +50,6 @@ __global__ void __launch_bounds__(kST) k_mul3(double *y, const double *a, const 
   if (t < n) y[t] = a[t] * b[t];
 }
 
-// y = y + a*b (the product rounded first, as multiply then add)
-__global__ void __launch_bounds__(kST) k_addmul(double *y, const double *a, const double *b, size_t n) {
-  const size_t t = (size_t)blockIdx.x * kST + threadIdx.x;
-  if (t < n) {
-    const double p = a[t] * b[t];
-    y[t] = y[t] + p;
-  }
-}
-
 // out = ((((F*1.5) + Fnm1*(-0.5)) + L) * dt), zero on the Dirichlet wall
 // planes of X (normal direction d, planes 1 and s_d-2 by mask), then + X.
 // has_L = 0 skips the + L (method 4).
@@ -123,15 +114,15 @@ struct moons_mhd_s {
   const moons_domain_s *dom = nullptr; // the fluid mesh inside mi (multi-domain only)
   moons_mhd_params P{};
   moons_field_s *U[3] = {}, *p = nullptr, *B[3] = {}, *phi = nullptr; // caller's
-  moons_field_s *Ustar[3] = {}, *F[3] = {}, *Fnm1[3] = {}, *L[3] = {}, *T1[3] = {}, *T2[3] = {}, *T3[3] = {};
-  moons_field_s *UE[6] = {}, *cc = nullptr, *tcc = nullptr;
-  moons_field_s *Bstar[3] = {}, *FB[3] = {}, *FBnm1[3] = {}, *LB[3] = {}, *B0[3] = {}, *J[3] = {}, *JxB[3] = {};
+  moons_field_s *Ustar[3] = {}, *F[3] = {}, *Fnm1[3] = {}, *T1[3] = {}, *T2[3] = {};
+  moons_field_s *UE[6] = {}, *tcc = nullptr;
+  moons_field_s *Bstar[3] = {}, *FB[3] = {}, *B0[3] = {}, *J[3] = {}, *JxB[3] = {};
   moons_field_s *Btot[3] = {}; // B0 (low Rem) or a field of its own, B0 + B (finite Rem)
-  moons_field_s *sig[3] = {}, *E[3] = {}, *ETF[6] = {}, *A6[6] = {}, *B6[6] = {};
+  moons_field_s *sig[3] = {}, *E[3] = {};
   // induction-mesh temporaries: U_E embedded (multi-domain only; else UE),
   // face temporaries (multi-domain only; else T1, T2) and the phi right-hand side
-  moons_field_s *UEi[6] = {}, *T1i[3] = {}, *T2i[3] = {}, *cci = nullptr, *tcci = nullptr;
-  bool own_i = false; // UEi, T1i, T2i, cci are fields of their own
+  moons_field_s *UEi[6] = {}, *T1i[3] = {}, *T2i[3] = {}, *tcci = nullptr;
+  bool own_i = false; // UEi, T1i, T2i are fields of their own
   moons_pcg_t pcg_p = nullptr, pcg_phi = nullptr;
   moons_pcgvf_t pcg_U = nullptr, pcg_B = nullptr;
   // buoyancy and gravity sources (caller's fields: T cell-centred, g three cell-centred components)
@@ -161,15 +152,13 @@ void mhd_free(moons_mhd_s *S) {
   if (S->P.finite_Rem)
     for (int d = 0; d < 3; ++d)
       if (S->Btot[d]) moons_field_destroy(S->Btot[d]);
-  moons_field_s **groups3[] = {S->Ustar, S->F, S->Fnm1, S->L, S->T1, S->T2, S->T3, S->Bstar, S->FB,
-                               S->FBnm1, S->LB, S->B0, S->J, S->JxB, S->sig, S->E};
+  moons_field_s **groups3[] = {S->Ustar, S->F, S->Fnm1, S->T1, S->T2, S->Bstar, S->FB, S->B0,
+                               S->J, S->JxB, S->sig, S->E};
   for (auto g : groups3)
     for (int d = 0; d < 3; ++d)
       if (g[d]) moons_field_destroy(g[d]);
-  moons_field_s **groups6[] = {S->UE, S->ETF, S->A6, S->B6};
-  for (auto g : groups6)
-    for (int q = 0; q < 6; ++q)
-      if (g[q]) moons_field_destroy(g[q]);
+  for (int q = 0; q < 6; ++q)
+    if (S->UE[q]) moons_field_destroy(S->UE[q]);
   if (S->own_i) {
     for (int q = 0; q < 6; ++q)
       if (S->UEi[q]) moons_field_destroy(S->UEi[q]);
@@ -177,10 +166,8 @@ void mhd_free(moons_mhd_s *S) {
       if (S->T1i[d]) moons_field_destroy(S->T1i[d]);
       if (S->T2i[d]) moons_field_destroy(S->T2i[d]);
     }
-    if (S->cci) moons_field_destroy(S->cci);
   }
   if (S->tcci) moons_field_destroy(S->tcci);
-  if (S->cc) moons_field_destroy(S->cc);
   if (S->tcc) moons_field_destroy(S->tcc);
   if (S->pcg_p) moons_pcg_destroy(S->pcg_p);
   if (S->pcg_phi) moons_pcg_destroy(S->pcg_phi);
@@ -203,92 +190,17 @@ int mul3(moons_field_s *y, const moons_field_s *a, const moons_field_s *b) {
   return MOONS_OK;
 }
 
-int addmul(moons_field_s *y, const moons_field_s *a, const moons_field_s *b) {
-  hipLaunchKernelGGL(k_addmul, dim3(sblk(y->n)), dim3(kST), 0, stream(), y->d, a->d, b->d, y->n);
-  MOONS_LAUNCH_CHECK();
-  return MOONS_OK;
-}
-
-// face i -> CC (along i) -> face j (along j)
-// face i -> CC (cc, a cell-centred temporary of u's mesh) -> face j
-int face2face(moons_field_s *cc, moons_field_s *out, const moons_field_s *u, int i, int j) {
-  int st;
-  if ((st = launch_interp(cc, u, i))) return st;
-  return launch_interp(out, cc, j);
-}
-
-// U_E = face2Edge_no_diag(U) (ops/ops_interp.f90:531-544)
-int face2edge_no_diag(moons_mhd_s *S) {
-  int st;
-  for (int q = 0; q < 6; ++q) {
-    const int i = kNoDiag[q][0], j = kNoDiag[q][1];
-    if ((st = launch_interp(S->UE[q], S->U[i], 3 - i - j))) return st;
-  }
-  return MOONS_OK;
-}
-
-// T1 = u_j d/dx_j u_i (advect_U_convection1, ops/ops_advect.f90:71-127)
-int convection(moons_mhd_s *S, moons_field_s *div[3]) {
-  int st;
-  for (int d = 0; d < 3; ++d) {
-    if ((st = launch_interp(S->cc, S->U[d], d))) return st;
-    if ((st = launch_del(S->T2[d], S->cc, 1, d, 0, 1))) return st;
-    if ((st = mul3(div[d], S->T2[d], S->U[d]))) return st;
-  }
-  // (U_E entry, derivative direction, velocity component), reference order
-  const int terms[3][2][3] = {{{4, 1, 1}, {2, 2, 2}}, {{5, 0, 0}, {0, 2, 2}}, {{3, 0, 0}, {1, 1, 1}}};
-  for (int d = 0; d < 3; ++d)
-    for (int t = 0; t < 2; ++t) {
-      const int q = terms[d][t][0], ddir = terms[d][t][1], vel = terms[d][t][2];
-      if ((st = launch_del(S->T2[d], S->UE[q], 1, ddir, 0, 1))) return st;
-      if ((st = face2face(S->cc, S->T3[d], S->U[vel], vel, d))) return st;
-      if ((st = addmul(div[d], S->T2[d], S->T3[d]))) return st;
-    }
-  return MOONS_OK;
-}
-
 int wall_mask(const moons_field_s *X, int d) {
   if (!X->has_bcs) return 0;
   return (X->bct[2 * d] == MOONS_BC_DIRICHLET ? 1 : 0) | (X->bct[2 * d + 1] == MOONS_BC_DIRICHLET ? 2 : 0);
 }
 
-int ab2_rhs(moons_field_s *out[3], moons_field_s *F[3], moons_field_s *Fnm1[3], moons_field_s *L[3],
-            moons_field_s *X[3], double dt, bool has_L) {
-  for (int d = 0; d < 3; ++d) {
-    const moons_field_s *x = X[d];
-    hipLaunchKernelGGL(k_ab2, dim3(sblk(x->n)), dim3(kST), 0, stream(), out[d]->d, F[d]->d, Fnm1[d]->d,
-                       has_L ? L[d]->d : F[d]->d, x->d, dt, x->s[0], x->s[1], x->s[2], d, wall_mask(x, d),
-                       has_L ? 1 : 0);
-    MOONS_LAUNCH_CHECK();
-  }
-  return MOONS_OK;
-}
-
 // J = curl(B)/Rem; Btot = B0 (+ B at finite Rem); JxB = N edge2Face(J) x face2Face(Btot)
 int post_induction(moons_mhd_s *S) {
   int st;
-  for (int d = 0; d < 3; ++d) {
-    if ((st = moons_curl(S->J[d], S->B[0], S->B[1], S->B[2], d))) return st;
-    if ((st = launch_scale(S->J[d], 1.0 / S->P.Rem))) return st;
-  }
-  if (S->P.finite_Rem)
-    for (int d = 0; d < 3; ++d) {
-      if ((st = moons_field_copy(S->Btot[d], S->B0[d]))) return st;
-      if ((st = axpy(S->Btot[d], S->B[d], 1.0))) return st; // B0 + B*1 = B0 + B exactly
-    }
-  for (int q = 0; q < 6; ++q) {
-    const int i = kNoDiag[q][0], j = kNoDiag[q][1];
-    if ((st = launch_interp(S->A6[q], S->J[i], 3 - i - j))) return st;  // edge2Face
-    if ((st = face2face(S->cci, S->B6[q], S->Btot[i], i, j))) return st;   // face2Face(Btot)
-  }
-  // (J x B)_x = J_y Bz - J_z By on x-faces; y negated form; z = J_x By - J_y Bx
-  if ((st = launch_cross(S->JxB[0], S->A6[0], S->B6[1], S->A6[1], S->B6[0], 1))) return st;
-  if ((st = launch_cross(S->JxB[1], S->A6[2], S->B6[3], S->A6[3], S->B6[2], -1))) return st;
-  if ((st = launch_cross(S->JxB[2], S->A6[4], S->B6[5], S->A6[5], S->B6[4], 1))) return st;
-  const double N = S->P.Ha * S->P.Ha / S->P.Re;
-  for (int d = 0; d < 3; ++d)
-    if ((st = launch_scale(S->JxB[d], N))) return st;
-  return MOONS_OK;
+  if ((st = launch_curl3(S->J, S->B, true, 1.0 / S->P.Rem))) return st;
+  if (S->P.finite_Rem && (st = launch_btot(S->Btot, S->B0, S->B))) return st;
+  return launch_jxb(S->JxB, S->J, S->Btot, S->P.Ha * S->P.Ha / S->P.Re);
 }
 
 int momentum(moons_mhd_s *S) {
@@ -302,54 +214,37 @@ int momentum(moons_mhd_s *S) {
     MOONS_LAUNCH_CHECK();
     if ((st = launch_apply_bcs3(S->U, false))) return st;
   }
-  for (int d = 0; d < 3; ++d) {
-    if ((st = moons_field_copy(S->Fnm1[d], S->F[d]))) return st;
-    if ((st = moons_field_fill(S->L[d], 0.0))) return st;
-    if ((st = moons_field_fill(S->F[d], 0.0))) return st;
+  // F = -convection (advect_U_convection1) + (1 - alpha)/Re lap(U) + J x B +
+  // buoyancy + gravity, and the right-hand side of U* (AB2)
+  MomSource M{};
+  M.U = S->U;
+  M.UE = S->UE;
+  M.F = S->F;
+  M.Fnm1 = S->Fnm1;
+  if (S->P.induction) {
+    // extract_add_JCrossB: the overlap of the induction mesh's J x B onto the
+    // fluid faces (every fluid face but the ghosts), ghosts zeroed
+    M.jx = S->dom ? S->T1 : S->JxB;
+    for (int d = 0; d < 3 && S->dom; ++d)
+      if ((st = launch_extract(S->T1[d], S->JxB[d], S->dom))) return st;
   }
-  if ((st = convection(S, S->T1))) return st;
-  for (int d = 0; d < 3; ++d)
-    if ((st = axpy(S->F[d], S->T1[d], -1.0))) return st;
-  const double ce = (1.0 / S->P.Re) * (1.0 - S->P.alpha_U);
-  for (int d = 0; d < 3; ++d) {
-    if ((st = launch_del(S->T1[d], S->U[d], 2, 0, 0, 1))) return st;
-    if ((st = launch_del(S->T1[d], S->U[d], 2, 1, 0, 2))) return st;
-    if ((st = launch_del(S->T1[d], S->U[d], 2, 2, 0, 2))) return st;
-    if ((st = axpy(S->F[d], S->T1[d], ce))) return st;
-  }
-  if (S->P.induction)
-    for (int d = 0; d < 3; ++d) {
-      // extract_add_JCrossB: the overlap of the induction mesh's J x B onto the
-      // fluid faces (every fluid face but the ghosts), ghosts zeroed
-      if ((st = S->dom ? launch_extract(S->T1[d], S->JxB[d], S->dom) : moons_field_copy(S->T1[d], S->JxB[d])))
-        return st;
-      if ((st = launch_assign_ghost_xperiodic(S->T1[d], 0.0))) return st;
-      if ((st = axpy(S->F[d], S->T1[d], 1.0))) return st;
-    }
-  if (S->add_buoy)
-    for (int d = 0; d < 3; ++d) {
-      // compute_add_buoyancy: temp_CC = T, times gravity, cellCenter2Face,
-      // extractFace (as J x B), F += buoyancy * scale
-      if ((st = mul3(S->tcc, S->Tb, S->grav[d]))) return st;
-      if ((st = launch_interp(S->T1[d], S->tcc, d))) return st;
-      if ((st = launch_assign_ghost_xperiodic(S->T1[d], 0.0))) return st;
-      if ((st = axpy(S->F[d], S->T1[d], S->buoy_scale))) return st;
-    }
-  if (S->add_grav)
-    for (int d = 0; d < 3; ++d) {
-      // compute_add_gravity: cellCenter2Face(g), extractFace, F += gravity * scale
-      if ((st = launch_interp(S->T1[d], S->grav[d], d))) return st;
-      if ((st = launch_assign_ghost_xperiodic(S->T1[d], 0.0))) return st;
-      if ((st = axpy(S->F[d], S->T1[d], S->grav_scale))) return st;
-    }
+  M.T = S->add_buoy ? S->Tb : nullptr;
+  M.g = S->grav;
+  M.grav = S->add_grav;
+  M.buoy_scale = S->buoy_scale;
+  M.grav_scale = S->grav_scale;
+  M.ce = (1.0 / S->P.Re) * (1.0 - S->P.alpha_U);
+  M.dt = S->P.dt;
+  for (int d = 0; d < 3; ++d) M.wall[d] = wall_mask(S->U[d], d);
   double scale;
   if (S->P.alpha_U == 0.0) {
-    if ((st = ab2_rhs(S->Ustar, S->F, S->Fnm1, S->L, S->U, S->P.dt, false))) return st;
+    M.rhs = S->Ustar;
+    if ((st = launch_mom_source(M))) return st;
     scale = 1.0;
   } else {
-    if ((st = ab2_rhs(S->T1, S->F, S->Fnm1, S->L, S->U, S->P.dt, true))) return st;
-    for (int d = 0; d < 3; ++d)
-      if ((st = moons_field_copy(S->Ustar[d], S->U[d]))) return st;
+    M.rhs = S->T1;
+    M.Ustar = S->Ustar;
+    if ((st = launch_mom_source(M))) return st;
     if ((st = moons_pcg_vf_update_mfp(S->pcg_U, S->P.dt * 1.0 * (-(1.0 / S->P.Re) * S->P.alpha_U), 1))) return st;
     if ((st = moons_pcg_vf_solve(S->pcg_U, S->Ustar, S->T1, &info))) return st;
     S->iters[0] = info.iterations;
@@ -357,32 +252,21 @@ int momentum(moons_mhd_s *S) {
   }
   if ((st = moons_clean_div(S->pcg_p, S->U, S->Ustar, S->p, scale, S->T2, S->tcc, &info))) return st;
   S->iters[1] = info.iterations;
-  return face2edge_no_diag(S);
+  return launch_face2edge(S->UE, S->U); // U_E = face2Edge_no_diag(U)
 }
 
 int induction(moons_mhd_s *S) {
   int st;
   moons_pcg_info info;
-  for (int d = 0; d < 3; ++d) {
-    if ((st = moons_field_copy(S->FBnm1[d], S->FB[d]))) return st;
-    if ((st = moons_field_fill(S->LB[d], 0.0))) return st;
-    if ((st = moons_field_fill(S->FB[d], 0.0))) return st;
-  }
   if (S->dom) // embedVelocity_E: the fluid's edge velocity into the induction mesh
     for (int q = 0; q < 6; ++q)
       if ((st = launch_embed(S->UEi[q], S->UE[q], S->dom))) return st;
-  if ((st = moons_advect_B(S->T1i, S->UEi, S->Btot, S->ETF, S->E))) return st;
-  for (int d = 0; d < 3; ++d)
-    if ((st = axpy(S->FB[d], S->T1i[d], 1.0))) return st;
-  for (int d = 0; d < 3; ++d)
-    if ((st = mul3(S->E[d], S->J[d], S->sig[d]))) return st;
-  for (int d = 0; d < 3; ++d) {
-    if ((st = moons_curl(S->T2i[d], S->E[0], S->E[1], S->E[2], d))) return st;
-    if ((st = axpy(S->FB[d], S->T2i[d], -0.0))) return st; // -beta, beta = 1 - alpha = 0
-  }
-  if ((st = ab2_rhs(S->T1i, S->FB, S->FBnm1, S->LB, S->B, S->P.dt, true))) return st;
-  for (int d = 0; d < 3; ++d)
-    if ((st = moons_field_copy(S->Bstar[d], S->B[d]))) return st;
+  // E = U_E x face2Edge(Btot); FB = curl(E) - (1 - alpha) curl(J sig), alpha = 1;
+  // the right-hand side of B* (AB2), and B* = B
+  int wall[3];
+  for (int d = 0; d < 3; ++d) wall[d] = wall_mask(S->B[d], d);
+  if ((st = launch_edge_cross(S->E, S->UEi, S->Btot, nullptr))) return st;
+  if ((st = launch_ind_source(S->E, S->J, S->sig, S->FB, S->B, S->T1i, S->Bstar, wall, S->P.dt))) return st;
   if ((st = moons_pcg_vf_update_mfp(S->pcg_B, S->P.dt * 1.0 * (1.0 / S->P.Rem), 1))) return st;
   if ((st = moons_pcg_vf_solve(S->pcg_B, S->Bstar, S->T1i, &info))) return st;
   S->iters[2] = info.iterations;
@@ -438,13 +322,12 @@ int moons_mhd_create_md(moons_mesh_t m, moons_mesh_t mi, moons_domain_t dom, con
   for (int d = 0; d < 3 && !st; ++d) {
     S->U[d] = U[d];
     if (P->induction) S->B[d] = B[d];
-    moons_field_s **vecs[] = {S->Ustar, S->F, S->Fnm1, S->L, S->T1, S->T2, S->T3};
+    moons_field_s **vecs[] = {S->Ustar, S->F, S->Fnm1, S->T1, S->T2};
     for (auto v : vecs)
       if (!st) st = fcreate(m, 1 << d, &v[d]);
     if (!st) copy_bcs_of(S->Ustar[d], U[d]);
   }
   for (int q = 0; q < 6 && !st; ++q) st = fcreate(m, kEdgeDL[kNoDiag[q][1]], &S->UE[q]);
-  if (!st) st = fcreate(m, MOONS_DL_CC, &S->cc);
   if (!st) st = fcreate(m, MOONS_DL_CC, &S->tcc);
   if (!st) {
     for (int d = 0; d < 3; ++d) st = st ? st : moons_field_fill(S->F[d], 0.0);
@@ -457,7 +340,7 @@ int moons_mhd_create_md(moons_mesh_t m, moons_mesh_t mi, moons_domain_t dom, con
   }
   if (!st && P->induction) {
     for (int d = 0; d < 3 && !st; ++d) {
-      moons_field_s **vecs[] = {S->Bstar, S->FB, S->FBnm1, S->LB, S->B0, S->JxB};
+      moons_field_s **vecs[] = {S->Bstar, S->FB, S->B0, S->JxB};
       for (auto v : vecs)
         if (!st) st = fcreate(mi, 1 << d, &v[d]);
       if (!st) copy_bcs_of(S->Bstar[d], B[d]);
@@ -473,21 +356,12 @@ int moons_mhd_create_md(moons_mesh_t m, moons_mesh_t mi, moons_domain_t dom, con
       if (!st) st = sigma_inv ? moons_field_copy(S->sig[d], sigma_inv[d]) : moons_field_fill(S->sig[d], 1.0);
       if (!st) st = fcreate(mi, kEdgeDL[d], &S->E[d]);
     }
-    // temp_E_TF of advect_B: Bx@y, Bx@z, By@x, By@z, Bz@x, Bz@y edges
-    const int etf_edge[6] = {1, 2, 0, 2, 0, 1};
-    for (int q = 0; q < 6 && !st; ++q) st = fcreate(mi, kEdgeDL[etf_edge[q]], &S->ETF[q]);
-    for (int q = 0; q < 6 && !st; ++q) {
-      st = fcreate(mi, 1 << kNoDiag[q][1], &S->A6[q]);
-      if (!st) st = fcreate(mi, 1 << kNoDiag[q][1], &S->B6[q]);
-    }
     if (!st) st = fcreate(mi, MOONS_DL_CC, &S->tcci);
     S->own_i = mi != m;
     for (int q = 0; q < 6 && !st; ++q) {
       if (!S->own_i) S->UEi[q] = S->UE[q];
       else if (!(st = fcreate(mi, kEdgeDL[kNoDiag[q][1]], &S->UEi[q]))) st = moons_field_fill(S->UEi[q], 0.0);
     }
-    if (!S->own_i) S->cci = S->cc;
-    else if (!st) st = fcreate(mi, MOONS_DL_CC, &S->cci);
     for (int d = 0; d < 3 && !st; ++d) {
       if (!S->own_i) {
         S->T1i[d] = S->T1[d];
@@ -504,7 +378,7 @@ int moons_mhd_create_md(moons_mesh_t m, moons_mesh_t mi, moons_domain_t dom, con
     if (!st) st = moons_pcg_set_isp(S->pcg_phi, P->iter_max[3], P->tol_rel[3], P->tol_abs[3], P->n_skip[3]);
     if (!st) st = post_induction(S);
   }
-  if (!st) st = face2edge_no_diag(S);
+  if (!st) st = launch_face2edge(S->UE, S->U);
   if (!st && (hipEventCreate(&S->ev0) != hipSuccess || hipEventCreate(&S->ev1) != hipSuccess))
     st = fail(MOONS_ERR_HIP, "moons_mhd_create: event creation failed");
   if (st) {
