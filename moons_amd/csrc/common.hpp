@@ -239,4 +239,13 @@ struct MomSource {
   double ce, dt, buoy_scale, grav_scale;
 };
 int launch_mom_source(const MomSource &S);
+// The energy equation's sources; UCC and q are scratch (KE diffusion, viscous
+// dissipation), qv the volumetric heating.
+struct NrgSource {
+  moons_field_s *const *U, *const *UCC, *const *J;
+  moons_field_s *T, *F, *Fnm1, *L, *q, *sig, *qv;
+  int advection, diffusion, diffusion_in_L, KE, viscous, joule, volumetric;
+  double c_adv, c_diff, c_KE, c_visc, c_joule, c_vol;
+};
+int launch_nrg_source(const NrgSource &S);
 }

@@ -44,39 +44,15 @@ __global__ void __launch_bounds__(kST) k_adds(double *y, double s, size_t n) {
   if (t < n) y[t] = y[t] + s;
 }
 
-// y = a*b
-__global__ void __launch_bounds__(kST) k_mul3(double *y, const double *a, const double *b, size_t n) {
-  const size_t t = (size_t)blockIdx.x * kST + threadIdx.x;
-  if (t < n) y[t] = a[t] * b[t];
-}
-
-// out = ((((F*1.5) + Fnm1*(-0.5)) + L) * dt), zero on the Dirichlet wall
-// planes of X (normal direction d, planes 1 and s_d-2 by mask), then + X.
-// has_L = 0 skips the + L (method 4).
-__global__ void __launch_bounds__(kST) k_ab2(double *out, const double *F, const double *Fnm1, const double *L,
-                                            const double *X, double dt, int s0, int s1, int s2, int d, int wall_mask,
-                                            int has_L) {
-  const size_t n = (size_t)s0 * s1 * s2;
+// out = (F*1.5 + Fnm1*(-0.5)) * dt + X
+__global__ void __launch_bounds__(kST) k_ab2(double *out, const double *F, const double *Fnm1, const double *X, double dt,
+                                            size_t n) {
   const size_t t = (size_t)blockIdx.x * kST + threadIdx.x;
   if (t >= n) return;
   double v = F[t] * 1.5;
   v = v + Fnm1[t] * (-0.5);
-  if (has_L) v = v + L[t];
   v = v * dt;
-  const int i = (int)(t % s0), j = (int)((t / s0) % s1), k = (int)(t / ((size_t)s0 * s1));
-  const int ii = d == 0 ? i : (d == 1 ? j : k);
-  const int sd = d == 0 ? s0 : (d == 1 ? s1 : s2);
-  if (((wall_mask & 1) && ii == 1) || ((wall_mask & 2) && ii == sd - 2)) v = 0.0;
   out[t] = v + X[t];
-}
-
-// acc = x*x (first) or acc + x*x: a left-to-right sum of squares over
-// successive launches, as square() then add() of the reference's fields
-__global__ void __launch_bounds__(kST) k_sqacc(double *acc, const double *x, int first, size_t n) {
-  const size_t t = (size_t)blockIdx.x * kST + threadIdx.x;
-  if (t >= n) return;
-  const double q = x[t] * x[t];
-  acc[t] = first ? q : acc[t] + q;
 }
 
 // O2_BDF_time_AB2_sources_SF's right-hand side (time_marching_methods_SF.f90:61-65):
@@ -176,18 +152,6 @@ void mhd_free(moons_mhd_s *S) {
   if (S->ev0) (void)hipEventDestroy(S->ev0);
   if (S->ev1) (void)hipEventDestroy(S->ev1);
   delete S;
-}
-
-int axpy(moons_field_s *y, const moons_field_s *x, double s) {
-  hipLaunchKernelGGL(k_axpy, dim3(sblk(y->n)), dim3(kST), 0, stream(), y->d, x->d, s, y->n);
-  MOONS_LAUNCH_CHECK();
-  return MOONS_OK;
-}
-
-int mul3(moons_field_s *y, const moons_field_s *a, const moons_field_s *b) {
-  hipLaunchKernelGGL(k_mul3, dim3(sblk(y->n)), dim3(kST), 0, stream(), y->d, a->d, b->d, y->n);
-  MOONS_LAUNCH_CHECK();
-  return MOONS_OK;
 }
 
 int wall_mask(const moons_field_s *X, int d) {
@@ -513,7 +477,7 @@ struct moons_nrg_s {
   moons_field_s *T = nullptr, *U[3] = {}; // caller's
   moons_field_s *J[3] = {}, *sig = nullptr; // caller's (Joule heating)
   moons_field_s *F = nullptr, *Fnm1 = nullptr, *L = nullptr, *Tnm1 = nullptr, *rhs = nullptr, *tcc = nullptr,
-                *tcc2 = nullptr, *tF[3] = {}, *UCC[3] = {}, *qv = nullptr;
+                *UCC[3] = {}, *qv = nullptr;
   moons_pcg_t pcg = nullptr;
   int iters = 0;
   int stage = 0; // RK stage (0-based) of the running step
@@ -531,8 +495,8 @@ constexpr double kRKAlpha[3] = {4.0 / 15.0, 1.0 / 15.0, 1.0 / 6.0};
 bool rk_active(const moons_nrg_s *S) { return S->P.rk_stages == 3; }
 
 void nrg_free(moons_nrg_s *S) {
-  moons_field_s *fs[] = {S->F,     S->Fnm1,   S->L,      S->Tnm1,   S->rhs,    S->tcc,    S->tcc2,
-                         S->tF[0], S->tF[1],  S->tF[2],  S->UCC[0], S->UCC[1], S->UCC[2], S->qv};
+  moons_field_s *fs[] = {S->F,     S->Fnm1,   S->L,      S->Tnm1,   S->rhs,    S->tcc,
+                         S->UCC[0], S->UCC[1], S->UCC[2], S->qv};
   for (auto f : fs)
     if (f) moons_field_destroy(f);
   if (S->pcg) moons_pcg_destroy(S->pcg);
@@ -541,80 +505,37 @@ void nrg_free(moons_nrg_s *S) {
   delete S;
 }
 
-int sqacc(moons_field_s *acc, const moons_field_s *x, bool first) {
-  hipLaunchKernelGGL(k_sqacc, dim3(sblk(acc->n)), dim3(kST), 0, stream(), acc->d, x->d, first ? 1 : 0, acc->n);
-  MOONS_LAUNCH_CHECK();
-  return MOONS_OK;
-}
-
-// lapUniformCoeff_SF (ops/ops_discrete.f90:101-110): collocated second
-// derivatives along x (assign), y and z (add)
-int lap_uniform(moons_field_s *out, const moons_field_s *f) {
-  int st;
-  if ((st = launch_del(out, f, 2, 0, 0, 1))) return st;
-  if ((st = launch_del(out, f, 2, 1, 0, 2))) return st;
-  return launch_del(out, f, 2, 2, 0, 2);
-}
-
 // add_all_energy_sources (solvers/energy/add_all_energy_sources.f90:21-80)
 int nrg_sources(moons_nrg_s *S) {
-  int st;
-  if ((st = moons_field_copy(S->Fnm1, S->F))) return st;
-  if (rk_active(S) && (st = moons_field_fill(S->L, 0.0))) return st;
-  if ((st = moons_field_fill(S->F, 0.0))) return st;
-  if (S->P.advection) {
-    // temp_F = cellCenter2Face(T); temp_F = temp_F * U; temp_CC = div(temp_F);
-    // temp_CC = -temp_CC; F = F + temp_CC * scale (the negation is exact, so
-    // it folds into the scale: (-t) s == t (-s) bit for bit)
-    for (int d = 0; d < 3; ++d) {
-      if ((st = launch_interp(S->tF[d], S->T, d))) return st;
-      hipLaunchKernelGGL(k_mul3, dim3(sblk(S->tF[d]->n)), dim3(kST), 0, stream(), S->tF[d]->d, S->tF[d]->d,
-                         S->U[d]->d, S->tF[d]->n);
-      MOONS_LAUNCH_CHECK();
-    }
-    if ((st = moons_div(S->tcc, S->tF[0], S->tF[1], S->tF[2]))) return st;
-    if ((st = axpy(S->F, S->tcc, -S->P.advection_scale))) return st;
-  }
-  if (S->P.diffusion) {
-    if ((st = lap_uniform(S->tcc, S->T))) return st;
-    if ((st = axpy(rk_active(S) ? S->L : S->F, S->tcc, S->P.diffusion_scale))) return st;
-  }
-  if (S->P.KE_diffusion || S->P.viscous_dissipation) // U_CC = face2CellCenter(U)
-    for (int d = 0; d < 3; ++d)
-      if ((st = launch_interp(S->UCC[d], S->U[d], d))) return st;
-  if (S->P.KE_diffusion) {
-    // temp_CC1 = Ux^2 + Uy^2 + Uz^2; temp_CC2 = lap(temp_CC1); F += temp_CC2 * scale
-    for (int d = 0; d < 3; ++d)
-      if ((st = sqacc(S->tcc, S->UCC[d], d == 0))) return st;
-    if ((st = lap_uniform(S->tcc2, S->tcc))) return st;
-    if ((st = axpy(S->F, S->tcc2, S->P.KE_diffusion_scale))) return st;
-  }
-  if (S->P.viscous_dissipation) {
-    // grad_TF (ops_discrete.f90:313-321): G[c][e] = d U_c / d x_e collocated
-    // on the cell centres; summed squared in add_SF_TF's order (TF_extend.f90:248-255):
-    // G[x][x], G[y][x], G[z][x], G[x][y], ..., G[z][z]
-    for (int e = 0; e < 3; ++e)
-      for (int c = 0; c < 3; ++c) {
-        if ((st = launch_del(S->tcc2, S->UCC[c], 1, e, 0, 1))) return st;
-        if ((st = sqacc(S->tcc, S->tcc2, e == 0 && c == 0))) return st;
-      }
-    if ((st = axpy(S->F, S->tcc, S->P.viscous_dissipation_scale))) return st;
-  }
-  if (S->P.joule_heating) {
-    if (!S->J[0] || !S->sig) return fail(MOONS_ERR_STATE, "moons_nrg_step: Joule heating needs moons_nrg_set_joule");
-    // edge2CellCenter_VF (ops_interp.f90:688-696): component d goes edge ->
-    // face fd = d+1 mod 3 along the third direction, then -> cell centre along fd
-    for (int d = 0; d < 3; ++d) {
-      const int fd = (d + 1) % 3, od = 3 - d - fd;
-      if ((st = launch_interp(S->tF[fd], S->J[d], od))) return st;
-      if ((st = launch_interp(S->tcc2, S->tF[fd], fd))) return st;
-      if ((st = sqacc(S->tcc, S->tcc2, d == 0))) return st;
-    }
-    if ((st = mul3(S->tcc, S->tcc, S->sig))) return st; // multiply(temp_CC, sigmaInv_CC)
-    if ((st = axpy(S->F, S->tcc, S->P.joule_heating_scale))) return st;
-  }
-  if (S->P.volumetric_heating && (st = axpy(S->F, S->qv, S->P.volumetric_heating_scale))) return st;
-  return MOONS_OK;
+  if (S->P.joule_heating && (!S->J[0] || !S->sig))
+    return fail(MOONS_ERR_STATE, "moons_nrg_step: Joule heating needs moons_nrg_set_joule");
+  NrgSource N{};
+  N.U = S->U;
+  N.UCC = S->UCC;
+  N.J = S->J;
+  N.T = S->T;
+  N.F = S->F;
+  N.Fnm1 = S->Fnm1;
+  N.L = S->L;
+  N.q = S->tcc;
+  N.sig = S->sig;
+  N.qv = S->qv;
+  N.advection = S->P.advection;
+  N.diffusion = S->P.diffusion;
+  N.diffusion_in_L = rk_active(S);
+  N.KE = S->P.KE_diffusion;
+  N.viscous = S->P.viscous_dissipation;
+  N.joule = S->P.joule_heating;
+  N.volumetric = S->P.volumetric_heating;
+  // temp_CC = -div(T U); F = F + temp_CC * scale: the negation is exact, so it
+  // folds into the scale, (-t) s == t (-s) bit for bit
+  N.c_adv = -S->P.advection_scale;
+  N.c_diff = S->P.diffusion_scale;
+  N.c_KE = S->P.KE_diffusion_scale;
+  N.c_visc = S->P.viscous_dissipation_scale;
+  N.c_joule = S->P.joule_heating_scale;
+  N.c_vol = S->P.volumetric_heating_scale;
+  return launch_nrg_source(N);
 }
 
 // solve_energy (governing_equations/energy_extend.f90:236-259), methods 1-5.
@@ -629,15 +550,13 @@ int nrg_march(moons_nrg_s *S) {
     return MOONS_OK;
   }
   if (S->P.method == 2) { // T = ((F*1.5 + Fnm1*(-0.5)) * dt) + T
-    hipLaunchKernelGGL(k_ab2, dim3(nb), dim3(kST), 0, stream(), S->T->d, S->F->d, S->Fnm1->d, (const double *)nullptr,
-                       S->T->d, dt, T->s[0], T->s[1], T->s[2], 0, 0, 0);
+    hipLaunchKernelGGL(k_ab2, dim3(nb), dim3(kST), 0, stream(), S->T->d, S->F->d, S->Fnm1->d, S->T->d, dt, T->n);
     MOONS_LAUNCH_CHECK();
     return MOONS_OK;
   }
   double c;
   if (S->P.method == 3) {
-    hipLaunchKernelGGL(k_ab2, dim3(nb), dim3(kST), 0, stream(), S->rhs->d, S->F->d, S->Fnm1->d,
-                       (const double *)nullptr, S->T->d, dt, T->s[0], T->s[1], T->s[2], 0, 0, 0);
+    hipLaunchKernelGGL(k_ab2, dim3(nb), dim3(kST), 0, stream(), S->rhs->d, S->F->d, S->Fnm1->d, S->T->d, dt, T->n);
     c = dt * 1.0 * S->P.coeff_implicit;
   } else if (S->P.method == 4) {
     const double two_thirds = 2.0 / 3.0, four_thirds = 4.0 / 3.0, neg_one_third = -1.0 / 3.0;
@@ -692,10 +611,9 @@ int moons_nrg_create(moons_mesh_t m, const moons_nrg_params *P, moons_field_t T,
   S->T = T;
   for (int d = 0; d < 3; ++d) S->U[d] = U ? U[d] : nullptr;
   int st = MOONS_OK;
-  moons_field_s **cc[] = {&S->F, &S->Fnm1, &S->L, &S->Tnm1, &S->rhs, &S->tcc, &S->tcc2};
+  moons_field_s **cc[] = {&S->F, &S->Fnm1, &S->L, &S->Tnm1, &S->rhs, &S->tcc};
   for (auto f : cc)
     if (!st) st = fcreate(m, MOONS_DL_CC, f);
-  for (int d = 0; d < 3 && !st; ++d) st = fcreate(m, 1 << d, &S->tF[d]);
   if (P->KE_diffusion || P->viscous_dissipation)
     for (int d = 0; d < 3 && !st; ++d) st = fcreate(m, MOONS_DL_CC, &S->UCC[d]);
   if (!st) st = moons_field_fill(S->F, 0.0);
