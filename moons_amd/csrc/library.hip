@@ -213,69 +213,84 @@ struct Shape3 {
   int s[3];
 };
 
-// One face of apply_BCs / apply_BCs_implicit over the full plane (tangential
-// ghosts included), raw rules of code/handwritten/BCs/direct/apply_BCs_faces_raw.f90
-// Up to three fields' faces of one direction (k_apply_bc_multi).
-struct BcMulti {
-  int on[3];
-  double *u[3];
-  Shape3 S[3];
-  int nalong[3];
-  int type[3][2];
-  double val[3][2], dh[3][2], r1[3][2], r2[3][2];
+// apply_BCs / apply_BCs_implicit of up to three fields in ONE launch, raw rules
+// of code/handwritten/BCs/direct/apply_BCs_faces_raw.f90 and
+// code/handwritten/BCs/implicit/apply_BCs_faces_raw_implicit.f90, which run
+// face after face (x, y, z; min, max) over full planes, tangential ghosts
+// included.  What bounds them is the launches: 4-5 us for each direction even
+// at 16^3, three for every vector and iteration of a vector solve.  No rule
+// reads a plane that a rule of its own direction writes, so an entry's final
+// value follows from entries that no rule writes: the z rule applied to values
+// after y, those from values after x (at most 8 reads, in an edge's corner).
+// Each thread forms one entry so, with the rules' roundings; an entry on
+// planes of several directions belongs to the last of them.
+// Three fields of a vector in a captured step of eight 16^3 to 96^3 states:
+// 3 x 4.4-5.2 us before, now 4.7-7.7.
+struct BcFace {
+  int type;
+  double val, dh, r1, r2; // r1, r2: the Robin coefficients of the rule applied (implicit: robi, 0)
+};
+struct BcField {
+  double *u;
+  int s[3];
+  int node[3];    // node-located along the direction
+  int planes[3];  // written planes along the direction
+  BcFace f[6];
+};
+struct BcArgs {
+  BcField x[3];
 };
 
-// and code/handwritten/BCs/implicit/apply_BCs_faces_raw_implicit.f90.
-// r1, r2: the face's Robin coefficients for the rule applied (implicit: robi, 0).
-__device__ __forceinline__ void apply_bc_point(double *u, const Shape3 &S, int face, int type, int nalong, double bval,
-                                               double dh_nhat, double r1, double r2, int implicit_, int ja, int jb) {
-  const int d = face / 2, is_max = face % 2;
-  const int a = (d + 1) % 3, b = (d + 2) % 3;
-  const int s = S.s[d];
-  int G, B, I, Io;
-  if (!nalong) {
-    G = is_max ? s - 1 : 0; B = -1; I = is_max ? s - 2 : 1; Io = is_max ? 1 : s - 2;
+// The planes a face's rule writes: its ghost plane (0 or s - 1); the wall plane
+// as well (node Dirichlet); the wall plane alone (node periodic, max face).
+__host__ __device__ __forceinline__ bool bc_writes(int type, int node, int side, int dist) {
+  if (type == MOONS_BC_NONE) return false;
+  if (node && type == MOONS_BC_DIRICHLET) return dist <= 1;
+  if (node && type == MOONS_BC_PERIODIC && side) return dist == 1;
+  return dist == 0;
+}
+__device__ __forceinline__ bool bc_written(const BcField &F, int d, int p) {
+  const int side = p >= F.s[d] / 2;
+  return bc_writes(side ? F.f[2 * d + 1].type : F.f[2 * d].type, F.node[d], side, side ? F.s[d] - 1 - p : p);
+}
+// The value of entry (q[0], q[1], q[2]) after the rules of directions 0 .. E.
+template <int E>
+__device__ __forceinline__ double bc_value(const BcField &F, const int (&q)[3], int implicit_) {
+  if constexpr (E < 0) {
+    return F.u[idx3(F.s, q[0], q[1], q[2])];
   } else {
-    G = is_max ? s - 1 : 0; B = is_max ? s - 2 : 1; I = is_max ? s - 3 : 2; Io = is_max ? 2 : s - 3;
-  }
-  int ii[3];
-  ii[a] = ja; ii[b] = jb;
-  ii[d] = G; const size_t ig = idx3(S.s, ii[0], ii[1], ii[2]);
-  ii[d] = I; const size_t iin = idx3(S.s, ii[0], ii[1], ii[2]);
-  switch (type) {
-    case MOONS_BC_DIRICHLET:
-      if (!nalong) {
-        u[ig] = implicit_ ? -u[iin] : 2.0 * bval - u[iin];
-      } else {
-        ii[d] = B; const size_t ib = idx3(S.s, ii[0], ii[1], ii[2]);
-        double ub = implicit_ ? 0.0 : bval;
-        u[ib] = ub;
-        u[ig] = implicit_ ? -u[iin] : 2.0 * ub - u[iin];
-      }
-      break;
-    case MOONS_BC_NEUMANN:
-      if (implicit_) u[ig] = u[iin];
-      else if (!nalong) u[ig] = u[iin] + bval * dh_nhat;
-      else u[ig] = u[iin] + 2.0 * bval * dh_nhat;
-      break;
-    case MOONS_BC_PERIODIC: {
-      int Gp = G, Iop = Io;
-      if (nalong && is_max && s > 4) { Gp = B; Iop = 1; }
-      ii[d] = Gp; const size_t igp = idx3(S.s, ii[0], ii[1], ii[2]);
-      ii[d] = Iop; const size_t io = idx3(S.s, ii[0], ii[1], ii[2]);
-      u[igp] = u[io];
-    } break;
-    case MOONS_BC_SYMMETRIC: u[ig] = u[iin]; break;
-    case MOONS_BC_ANTISYMMETRIC: u[ig] = -u[iin]; break;
-    case MOONS_BC_ROBIN:
-      if (!nalong) {
-        u[ig] = implicit_ ? u[iin] * r1 : u[iin] * r1 + bval * r2;
-      } else {
-        ii[d] = B; const size_t ib = idx3(S.s, ii[0], ii[1], ii[2]);
-        u[ig] = implicit_ ? u[iin] + u[ib] * r1 : u[iin] + u[ib] * r1 + bval * r2;
-      }
-      break;
-    default: break;
+    const int p = q[E], s = F.s[E], side = p >= s / 2, node = F.node[E];
+    // (selected, not indexed: the faces' constants are uniform and stay in scalar registers)
+    const BcFace &f0 = F.f[2 * E], &f1 = F.f[2 * E + 1];
+    const BcFace f{side ? f1.type : f0.type, side ? f1.val : f0.val, side ? f1.dh : f0.dh, side ? f1.r1 : f0.r1,
+                   side ? f1.r2 : f0.r2};
+    const bool on = bc_writes(f.type, node, side, side ? s - 1 - p : p);
+    const bool periodic = f.type == MOONS_BC_PERIODIC;
+    // the plane read: the first interior one, or (periodic) the opposite face's
+    const int in = node ? 2 : 1, side_r = periodic ? !side : side;
+    int r = side_r ? s - 1 - in : in;
+    if (periodic && node && side) r = 1;
+    int a[3] = {q[0], q[1], q[2]};
+    if (on) a[E] = r;
+    const double v = bc_value<E - 1>(F, a, implicit_);
+    if (!on) return v;
+    switch (f.type) {
+      case MOONS_BC_DIRICHLET:
+        if (node && p != (side ? s - 1 : 0)) return implicit_ ? 0.0 : f.val;
+        return implicit_ ? -v : 2.0 * f.val - v;
+      case MOONS_BC_NEUMANN:
+        if (implicit_) return v;
+        return node ? v + 2.0 * f.val * f.dh : v + f.val * f.dh;
+      case MOONS_BC_ANTISYMMETRIC: return -v;
+      case MOONS_BC_ROBIN:
+        if (!node) return implicit_ ? v * f.r1 : v * f.r1 + f.val * f.r2;
+        {
+          a[E] = side ? s - 2 : 1;
+          const double w = bc_value<E - 1>(F, a, implicit_);
+          return implicit_ ? v + w * f.r1 : v + w * f.r1 + f.val * f.r2;
+        }
+      default: return v; // periodic, symmetric
+    }
   }
 }
 
@@ -285,36 +300,35 @@ static inline void robin_pair(const BCDev &b, int face, bool implicit_, double &
   r2 = implicit_ ? 0.0 : b.rob2[face];
 }
 
-__global__ void __launch_bounds__(256) k_apply_bc_face(double *u, Shape3 S, int face, int type, int nalong,
-                                                       double bval, double dh_nhat, double r1, double r2,
-                                                       int implicit_, const int *gate) {
+__global__ void __launch_bounds__(256) k_apply_bcs(BcArgs A, int implicit_, const int *gate) {
   if (gate && *gate) return;
-  const int d = face / 2;
-  const int a = (d + 1) % 3, b = (d + 2) % 3;
-  const int na = S.s[a], nb = S.s[b];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= na * nb) return;
-  apply_bc_point(u, S, face, type, nalong, bval, dh_nhat, r1, r2, implicit_, t % na, t / na);
-}
-
-// Both faces of direction d in one launch: the first na*nb threads the min
-// face, the others the max face.  Used when the direction has at least 6
-// points, where the planes one face writes are none of those the other reads,
-// so the result equals the min-then-max sequence.
-__global__ void __launch_bounds__(256) k_apply_bc_pair(double *u, Shape3 S, int d, int type0, int type1, int nalong,
-                                                       double bval0, double bval1, double dh0, double dh1,
-                                                       double r10, double r11, double r20, double r21,
-                                                       int implicit_, const int *gate) {
-  if (gate && *gate) return;
-  const int a = (d + 1) % 3, b = (d + 2) % 3;
-  const int na = S.s[a], nb = S.s[b];
-  const int np = na * nb;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 2 * np) return;
-  const int side = t >= np ? 1 : 0;
-  const int q = t - side * np;
-  apply_bc_point(u, S, 2 * d + side, side ? type1 : type0, nalong, side ? bval1 : bval0, side ? dh1 : dh0,
-                 side ? r11 : r10, side ? r21 : r20, implicit_, q % na, q / na);
+  const BcField &F = A.x[blockIdx.y];
+  unsigned t = blockIdx.x * 256u + threadIdx.x;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int lo = d == 0 ? 1 : 0, hi = d == 2 ? 1 : 2;
+    const unsigned np = (unsigned)F.s[lo] * F.s[hi], n = np * F.planes[d];
+    if (t >= n) {
+      t -= n;
+      continue;
+    }
+    // the t / np -th written plane, from the min face on
+    int k = (int)(t / np), p = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int pl = c < 2 ? c : F.s[d] - 4 + c;
+      if (bc_written(F, d, pl) && k-- == 0) p = pl;
+    }
+    const unsigned r = t % np;
+    int q[3];
+    q[lo] = r % F.s[lo];
+    q[hi] = r / F.s[lo];
+    q[d] = p;
+    // written once, by the last direction whose planes hold it
+    if ((d < 1 && bc_written(F, 1, q[1])) || (d < 2 && bc_written(F, 2, q[2]))) return;
+    F.u[idx3(F.s, q[0], q[1], q[2])] = bc_value<2>(F, q, implicit_);
+    return;
+  }
 }
 
 // Assigns val to one whole plane idx along direction d.
@@ -554,98 +568,41 @@ __global__ void __launch_bounds__(256) k_volume(double *vol, Shape3 S, int e0, i
 // --------------------------------------------------------------- launchers
 static inline unsigned nblk(size_t n) { return (unsigned)((n + 255) / 256); }
 
-int launch_apply_bcs(moons_field_s *u, bool implicit_) {
-  if (!u->has_bcs) return MOONS_OK;
-  Shape3 S{{u->s[0], u->s[1], u->s[2]}};
-  BCDev b = make_bcdev(u);
-  for (int d = 0; d < 3; ++d) {
-    const int a = (d + 1) % 3, bb = (d + 2) % 3;
-    const size_t np = (size_t)u->s[a] * u->s[bb];
-    const int nalong = (u->dl >> d) & 1;
-    const int f0 = 2 * d, f1 = 2 * d + 1;
-    double r1[2], r2[2];
-    robin_pair(b, f0, implicit_, r1[0], r2[0]);
-    robin_pair(b, f1, implicit_, r1[1], r2[1]);
-    if (b.type[f0] != MOONS_BC_NONE && b.type[f1] != MOONS_BC_NONE && u->s[d] >= 6) {
-      hipLaunchKernelGGL(k_apply_bc_pair, dim3(nblk(2 * np)), dim3(256), 0, g_stream, u->d, S, d, b.type[f0],
-                         b.type[f1], nalong, b.val[f0], b.val[f1], b.dh_nhat[f0], b.dh_nhat[f1], r1[0], r1[1], r2[0],
-                         r2[1], implicit_ ? 1 : 0, g_gate);
-      MOONS_LAUNCH_CHECK();
-      continue;
-    }
-    for (int face : {f0, f1}) {
-      if (b.type[face] == MOONS_BC_NONE) continue;
-      hipLaunchKernelGGL(k_apply_bc_face, dim3(nblk(np)), dim3(256), 0, g_stream, u->d, S, face, b.type[face],
-                         nalong, b.val[face], b.dh_nhat[face], r1[face - f0], r2[face - f0], implicit_ ? 1 : 0,
-                         g_gate);
-      MOONS_LAUNCH_CHECK();
-    }
-  }
-  return MOONS_OK;
-}
-
-// apply_BCs of three fields: per direction, the faces of every field whose
-// direction has at least 6 points in one launch (fields are independent, so
-// only each field's own direction order matters), the others face by face.
-__global__ void __launch_bounds__(256) k_apply_bc_multi(BcMulti M, int d, int implicit_, const int *gate) {
-  if (gate && *gate) return;
-  const int f = blockIdx.y;
-  if (!M.on[f]) return;
-  const Shape3 &S = M.S[f];
-  const int a = (d + 1) % 3, b = (d + 2) % 3;
-  const int na = S.s[a], nb = S.s[b];
-  const int np = na * nb;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 2 * np) return;
-  const int side = t >= np ? 1 : 0;
-  const int q = t - side * np;
-  apply_bc_point(M.u[f], S, 2 * d + side, M.type[f][side], M.nalong[f], M.val[f][side], M.dh[f][side],
-                 M.r1[f][side], M.r2[f][side], implicit_, q % na, q / na);
-}
-
-int launch_apply_bcs3(moons_field_s *const u[3], bool implicit_) {
-  for (int d = 0; d < 3; ++d) {
-    BcMulti M{};
-    size_t npmax = 0;
-    for (int f = 0; f < 3; ++f) {
-      const moons_field_s *x = u[f];
-      if (!x->has_bcs) continue;
-      BCDev b = make_bcdev(x);
-      const int f0 = 2 * d, f1 = 2 * d + 1;
-      const int a = (d + 1) % 3, bb = (d + 2) % 3;
-      const size_t np = (size_t)x->s[a] * x->s[bb];
-      if (b.type[f0] != MOONS_BC_NONE && b.type[f1] != MOONS_BC_NONE && x->s[d] >= 6) {
-        M.on[f] = 1;
-        M.u[f] = x->d;
-        M.S[f] = Shape3{{x->s[0], x->s[1], x->s[2]}};
-        M.nalong[f] = (x->dl >> d) & 1;
-        for (int side = 0; side < 2; ++side) {
-          M.type[f][side] = b.type[2 * d + side];
-          M.val[f][side] = b.val[2 * d + side];
-          M.dh[f][side] = b.dh_nhat[2 * d + side];
-          robin_pair(b, 2 * d + side, implicit_, M.r1[f][side], M.r2[f][side]);
-        }
-        npmax = std::max(npmax, np);
-      } else {
-        Shape3 S{{x->s[0], x->s[1], x->s[2]}};
-        for (int face : {f0, f1}) {
-          if (b.type[face] == MOONS_BC_NONE) continue;
-          double r1, r2;
-          robin_pair(b, face, implicit_, r1, r2);
-          hipLaunchKernelGGL(k_apply_bc_face, dim3(nblk(np)), dim3(256), 0, g_stream, x->d, S, face, b.type[face],
-                             (x->dl >> d) & 1, b.val[face], b.dh_nhat[face], r1, r2, implicit_ ? 1 : 0, g_gate);
-          MOONS_LAUNCH_CHECK();
-        }
+static int apply_bcs(moons_field_s *const *u, int nf, bool implicit_) {
+  BcArgs A{};
+  size_t nmax = 0;
+  int on = 0;
+  for (int q = 0; q < nf; ++q) {
+    const moons_field_s *x = u[q];
+    if (!x->has_bcs) continue;
+    const BCDev b = make_bcdev(x);
+    BcField &F = A.x[on++];
+    F.u = x->d;
+    size_t n = 0;
+    for (int d = 0; d < 3; ++d) {
+      F.s[d] = x->s[d];
+      F.node[d] = (x->dl >> d) & 1;
+      for (int side = 0; side < 2; ++side) {
+        BcFace &f = F.f[2 * d + side];
+        f.type = b.type[2 * d + side];
+        f.val = b.val[2 * d + side];
+        f.dh = b.dh_nhat[2 * d + side];
+        robin_pair(b, 2 * d + side, implicit_, f.r1, f.r2);
+        for (int dist = 0; dist < 2; ++dist) F.planes[d] += bc_writes(f.type, F.node[d], side, dist) ? 1 : 0;
       }
+      n += (size_t)F.planes[d] * x->s[(d + 1) % 3] * x->s[(d + 2) % 3];
     }
-    if (npmax > 0) {
-      hipLaunchKernelGGL(k_apply_bc_multi, dim3(nblk(2 * npmax), 3), dim3(256), 0, g_stream, M, d, implicit_ ? 1 : 0,
-                         g_gate);
-      MOONS_LAUNCH_CHECK();
-    }
+    if (n >= (size_t)1 << 31) return fail(MOONS_ERR_ARG, "apply_BCs: planes of 2^31 or more elements are not supported");
+    nmax = std::max(nmax, n);
   }
+  if (nmax == 0) return MOONS_OK;
+  hipLaunchKernelGGL(k_apply_bcs, dim3(nblk(nmax), on), dim3(256), 0, g_stream, A, implicit_ ? 1 : 0, g_gate);
+  MOONS_LAUNCH_CHECK();
   return MOONS_OK;
 }
+
+int launch_apply_bcs(moons_field_s *u, bool implicit_) { return apply_bcs(&u, 1, implicit_); }
+int launch_apply_bcs3(moons_field_s *const u[3], bool implicit_) { return apply_bcs(u, 3, implicit_); }
 
 int launch_assign_ghost_xperiodic(moons_field_s *u, double val) {
   int mask = 0;

@@ -7,7 +7,7 @@
 // 176-202) and prec_mom_VF / prec_ind_VF (preconditioners.f90:86-129).
 //
 // One iteration, all on the three components at once (one grid row each):
-//   apply_BCs_implicit(p)   a launch per direction
+//   apply_BCs_implicit(p)   one launch
 //   k_vf_mom_op | k_vf_curl twice   Ax = vol A p with the wall rules
 //   k_vf_dot       partials of (p,Ax)
 //   k_vf_update    alpha; x += a p, r -= a Ax, partials (r,r), (Minv r, r)

@@ -62,3 +62,28 @@ def test_div_is_three_del_passes(gpu, n, periodic):
         if d != periodic:
             np.moveaxis(want, d, 0)[[0, -1]] = 0.0
     np.testing.assert_array_equal(out.download(), want)
+
+
+BC_SETS = [
+    (["Dirichlet", "Neumann", "Neumann", "Dirichlet", "Robin", "Symmetric"], [0.3, -0.2, 0.7, 1.0, 0.5, 0.1]),
+    (["Periodic", "Periodic", "Robin", "Robin", "Antisymmetric", "Dirichlet"], [0, 0, 0.2, -0.4, 0.1, 0.6]),
+    (["Robin", "Dirichlet", "Periodic", "Periodic", "Periodic", "Periodic"], [0.4, 1.5, 0, 0, 0, 0]),
+    (["none", "Dirichlet", "Neumann", "none", "none", "none"], [0, 0.3, 0.2, 0, 0, 0]),
+]
+
+
+@pytest.mark.parametrize("n", SHAPES)
+@pytest.mark.parametrize("bc", range(len(BC_SETS)))
+@pytest.mark.parametrize("implicit", [False, True])
+def test_apply_bcs_sizes(gpu, n, bc, implicit):
+    """Every face's rule in one launch: edges and corners as the face sequence leaves them."""
+    g, m = _grid(gpu, n)
+    types, vals = BC_SETS[bc]
+    cw = [0.01, 0.02, 0.5, 1.0, 3.0, 0.07]
+    for dl in range(8):
+        u = _rand(g.shape(dl), 30 + dl)
+        ref = u.copy(order="F")
+        O.apply_bcs(g, ref, dl, O.BCs.make(types, vals, cw), implicit)
+        U = gpu.SF(m, dl).upload(u).set_BCs(types, vals, c_w=cw)
+        (gpu.apply_BCs_implicit if implicit else gpu.apply_BCs)(U)
+        np.testing.assert_array_equal(U.download(), ref, err_msg=f"dl={dl}")
