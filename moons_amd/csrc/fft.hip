@@ -13,10 +13,10 @@
 // (ops_idct.f90: x(j) = Y(1)/N + 2/N sum_{k>=2} Y(k) cos(...)) gives u's
 // interior, and u's BCs set its ghosts.
 //
-// On the GPU each transform along one direction is one FP64 GEMM with the
-// N x N cosine matrix (rocBLAS, on the matrix cores): along x the matrix
-// multiplies the n0 x (n1 n2) view from the left, along y a strided batch of
-// n0 x n1 planes from the right, along z the (n0 n1) x n2 view from the right.
+// On the GPU each transform along one direction is an FP64 GEMM with the
+// N x N cosine matrix (rocBLAS, on the matrix cores), a strided batch of planes:
+// along x the matrix multiplies the n0 x n1 planes from the left, along y from
+// the right, along z the n0 x n2 planes from the right.
 // The reference computes the same transforms with a radix-2 FFT, so the two
 // agree to rounding.
 //
@@ -56,16 +56,7 @@ namespace {
 
 constexpr int kFT = 256;
 
-// compact interior <- padded field, and back
-__global__ void __launch_bounds__(kFT) k_fft_pack(const double *__restrict__ f, double *__restrict__ w, int n0, int n1,
-                                                  int n2) {
-  const long long t = (long long)blockIdx.x * kFT + threadIdx.x;
-  const long long nc = (long long)n0 * n1 * n2;
-  if (t >= nc) return;
-  const int i = (int)(t % n0), j = (int)((t / n0) % n1), k = (int)(t / ((long long)n0 * n1));
-  w[t] = f[(size_t)(i + 1) + (size_t)(n0 + 2) * ((size_t)(j + 1) + (size_t)(n1 + 2) * (size_t)(k + 1))];
-}
-
+// padded field <- compact interior
 __global__ void __launch_bounds__(kFT) k_fft_unpack(const double *__restrict__ w, double *__restrict__ u, int n0,
                                                     int n1, int n2) {
   const long long t = (long long)blockIdx.x * kFT + threadIdx.x;
@@ -93,22 +84,41 @@ unsigned fblocks(long long n) { return (unsigned)((n + kFT - 1) / kFT); }
 
 const char *blas_msg(rocblas_status s) { return rocblas_status_to_string(s); }
 
+// A view of the n0 x n1 x n2 cells: first element and the strides of y and z
+// (a compact array, or the interior of a padded field).
+struct CellView {
+  double *p;
+  long long sy, sz;
+};
+
 // Y = transform of X along direction t with the n_t x n_t matrix M
-// (row = output index, column = input index, column-major).
-int transform(moons_fft_s *F, int t, const double *M, const double *X, double *Y) {
+// (row = output index, column = input index, column-major).  A product each
+// x-y plane (t = 0, 1) or x-z plane (t = 2) reads the padded right-hand side and
+// writes the padded solution without a copy into or out of a compact array (8-9
+// us each at 128^3), and fills the chip better than one product over a compact
+// array (14.7 against 21.3 us).  Planes too thin to fill a tile stay one
+// product: along x below 48 columns (160 x 33 x 20: 41 us a solve, 48 with a
+// product each plane), along z below 24 rows (12 x 160 x 160: 92 against 110).
+constexpr int kThinX = 48, kThinZ = 24;
+int transform(moons_fft_s *F, int t, const double *M, const CellView &X, const CellView &Y) {
   const int n0 = F->n[0], n1 = F->n[1], n2 = F->n[2];
   const double one = 1.0, zero = 0.0;
   rocblas_status s;
-  if (t == 0) {
-    s = rocblas_dgemm(F->blas, rocblas_operation_none, rocblas_operation_none, n0, n1 * n2, n0, &one, M, n0, X, n0,
-                      &zero, Y, n0);
+  if (t == 0 && n1 < kThinX && X.sy == n0 && Y.sy == n0) {
+    s = rocblas_dgemm(F->blas, rocblas_operation_none, rocblas_operation_none, n0, n1 * n2, n0, &one, M, n0, X.p, n0,
+                      &zero, Y.p, n0);
+  } else if (t == 0) {
+    s = rocblas_dgemm_strided_batched(F->blas, rocblas_operation_none, rocblas_operation_none, n0, n1, n0, &one, M, n0,
+                                      0, X.p, (int)X.sy, X.sz, &zero, Y.p, (int)Y.sy, Y.sz, n2);
   } else if (t == 1) {
     s = rocblas_dgemm_strided_batched(F->blas, rocblas_operation_none, rocblas_operation_transpose, n0, n1, n1, &one,
-                                      X, n0, (rocblas_stride)n0 * n1, M, n1, 0, &zero, Y, n0,
-                                      (rocblas_stride)n0 * n1, n2);
+                                      X.p, (int)X.sy, X.sz, M, n1, 0, &zero, Y.p, (int)Y.sy, Y.sz, n2);
+  } else if (n0 < kThinZ && X.sy == n0 && Y.sy == n0) {
+    s = rocblas_dgemm(F->blas, rocblas_operation_none, rocblas_operation_transpose, n0 * n1, n2, n2, &one, X.p, n0 * n1,
+                      M, n2, &zero, Y.p, n0 * n1);
   } else {
-    s = rocblas_dgemm(F->blas, rocblas_operation_none, rocblas_operation_transpose, n0 * n1, n2, n2, &one, X, n0 * n1,
-                      M, n2, &zero, Y, n0 * n1);
+    s = rocblas_dgemm_strided_batched(F->blas, rocblas_operation_none, rocblas_operation_transpose, n0, n2, n2, &one,
+                                      X.p, (int)X.sz, X.sy, M, n2, 0, &zero, Y.p, (int)Y.sz, Y.sy, n1);
   }
   if (s != rocblas_status_success) return fail(MOONS_ERR_HIP, std::string("DCT transform (rocBLAS dgemm): ") + blas_msg(s));
   return MOONS_OK;
@@ -233,21 +243,25 @@ int moons_fft_solve(moons_fft_t F, moons_field_t u, moons_field_t f) {
     return fail(MOONS_ERR_HIP, "moons_fft_solve: rocblas_set_stream failed");
   const int n0 = F->n[0], n1 = F->n[1], n2 = F->n[2];
   const long long nc = (long long)n0 * n1 * n2;
-  hipLaunchKernelGGL(k_fft_pack, dim3(fblocks(nc)), dim3(kFT), 0, stream(), f->d, F->W, n0, n1, n2);
-  MOONS_LAUNCH_CHECK();
+  const long long s0 = n0 + 2, s01 = s0 * (n1 + 2), first = 1 + s0 + s01;
+  const CellView W{F->W, n0, (long long)n0 * n1}, V{F->V, n0, (long long)n0 * n1};
+  const CellView fi{f->d + first, s0, s01}, ui{u->d + first, s0, s01};
   int st;
-  // forward: along a (W -> V), along b (V -> W)
-  if ((st = transform(F, F->a, F->C[F->a], F->W, F->V))) return st;
-  if ((st = transform(F, F->b, F->C[F->b], F->V, F->W))) return st;
+  // forward: along a (f -> V), along b (V -> W)
+  if ((st = transform(F, F->a, F->C[F->a], fi, V))) return st;
+  if ((st = transform(F, F->b, F->C[F->b], V, W))) return st;
   const int x_quirk = F->kind == MOONS_FFT_COEF_REFERENCE && F->dir == 0;
   hipLaunchKernelGGL(k_fft_scale, dim3(fblocks(nc)), dim3(kFT), 0, stream(), F->W, F->coef, n0, n1, n2, F->a, F->b,
                      x_quirk);
   MOONS_LAUNCH_CHECK();
-  // inverse: along a (W -> V), along b (V -> W)
-  if ((st = transform(F, F->a, F->Ci[F->a], F->W, F->V))) return st;
-  if ((st = transform(F, F->b, F->Ci[F->b], F->V, F->W))) return st;
-  hipLaunchKernelGGL(k_fft_unpack, dim3(fblocks(nc)), dim3(kFT), 0, stream(), F->W, u->d, n0, n1, n2);
-  MOONS_LAUNCH_CHECK();
+  // inverse: along a (W -> V), along b (V -> u; a thin z transform stays compact)
+  const bool thin = F->b == 2 && n0 < kThinZ;
+  if ((st = transform(F, F->a, F->Ci[F->a], W, V))) return st;
+  if ((st = transform(F, F->b, F->Ci[F->b], V, thin ? W : ui))) return st;
+  if (thin) {
+    hipLaunchKernelGGL(k_fft_unpack, dim3(fblocks(nc)), dim3(kFT), 0, stream(), F->W, u->d, n0, n1, n2);
+    MOONS_LAUNCH_CHECK();
+  }
   return launch_apply_bcs(u, false);
 }
 
