@@ -11,7 +11,7 @@
 //   restriction volume-weighted sum of the 8 children's residuals
 //   prolongation trilinear in the true cell-centre coordinates (stretched
 //               grids), coarse ghosts from the BC rule
-//   coarsest    one workgroup, a fixed number of red-black sweeps
+//   coarsest    a fixed number of red-black sweeps: in the LDS tail, or over the grid
 // Everything is FP32 (4 B/cell per array): this is the preconditioner of an
 // FP64 flexible PCG whose residual, dot products and BCs stay FP64.
 #include "mg.hpp"
@@ -141,20 +141,6 @@ __device__ __forceinline__ float res_cell(const LevelDev &L, int i, int j, int k
   s += d * x[lidx(L, i, j, k)];
   return L.f[lidx(L, i, j, k)] - s;
 }
-
-// Cells of one colour, (i+j+k) % 2 == color, one thread each.
-__device__ __forceinline__ bool color_cell(const LevelDev &L, long long t, int color, int &i, int &j, int &k) {
-  const int h0 = (L.n0 + 1) / 2;
-  const long long per_k = (long long)h0 * L.n1;
-  if (t >= per_k * L.n2) return false;
-  k = 1 + (int)(t / per_k);
-  const long long r = t % per_k;
-  j = 1 + (int)(r / h0);
-  const int ipair = (int)(r % h0);
-  i = 2 * ipair + 1 + ((color + j + k + 1) & 1);
-  return i <= L.n0;
-}
-
 
 // One half-sweep: the cells of one colour, (i+j+k) % 2 == color.  Thread x
 // of the tile is the pair index p of row (j, k), i.e. the cell of this colour
@@ -644,22 +630,6 @@ __global__ void __launch_bounds__(256) k_mg_prolong(LevelDev F, LevelDev C, int 
                                     by[cy] * (az[cz] * v[1][y2][x2] + bz[cz] * v[z2][y2][x2]));
           if (!skip) F.x[lidx(F, 2 * I - 1 + cx, 2 * J - 1 + cy, 2 * K - 1 + cz)] = xf[cz][cy][cx] + e;
         }
-  }
-}
-
-// Coarsest level: one workgroup, `sweeps` red-black sweeps from x = 0.
-__global__ void __launch_bounds__(1024) k_mg_coarse(LevelDev L, int sweeps, const int *done) {
-  if (done && *done) return;
-  const int h0 = (L.n0 + 1) / 2;
-  const long long ncol = (long long)h0 * L.n1 * L.n2;
-  for (int s = 0; s < sweeps; ++s) {
-    for (int color = 0; color < 2; ++color) {
-      for (long long t = threadIdx.x; t < ncol; t += blockDim.x) {
-        int i, j, k;
-        if (color_cell(L, t, color, i, j, k)) L.x[lidx(L, i, j, k)] = gs_cell(L, L.x, i, j, k, s == 0 && color == 0);
-      }
-      __syncthreads();
-    }
   }
 }
 
@@ -1384,6 +1354,23 @@ static void sweep(LevelDev &L, int c_first, bool zero_first, const int *done, in
   }
 }
 
+// Coarsest level that the LDS tail cannot hold (an odd count stops coarsening
+// early): a fixed number of red-black sweeps from x = 0 over the whole grid, a
+// launch a sweep (two beyond kFusedSweepMaxCells).  One workgroup doing them
+// with a barrier a colour gave the same values in 1.8 ms a V-cycle at 50 x 39 x 45 and
+// 42 ms at 160 x 160 x 75 (one level each, whole solve); now 0.13 and 0.31 ms.
+static void coarse_solve(LevelDev &L, int sweeps, const int *done) {
+  const bool fused = (long long)L.n0 * L.n1 * L.n2 <= kFusedSweepMaxCells;
+  for (int s = 0; s < sweeps; ++s) {
+    if (fused) {
+      sweep2(L, 0, s == 0, done);
+    } else {
+      smooth(L, 0, s == 0, done);
+      smooth(L, 1, false, done);
+    }
+  }
+}
+
 static void restrict_to(const LevelDev &F, const LevelDev &C, const int *done) {
   const TileLaunch t = tiles(C.n0, C.n1, C.n2);
   hipLaunchKernelGGL(k_mg_restrict, t.grid, t.block, 0, stream(), F, C, t.kz, done);
@@ -1470,7 +1457,7 @@ int mg_vcycle(MGHier *h, const int *done) {
       hipLaunchKernelGGL(k_mg_tail, dim3(1), dim3(kTailThreads), h->tail_lds, stream(), h->tailimg, h->tail,
                          nu1_at(g), nu2_at(g), h->coarse_sweeps, done);
     else
-      hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(1024), 0, stream(), h->L[nl - 1], h->coarse_sweeps, done);
+      coarse_solve(h->L[nl - 1], h->coarse_sweeps, done);
     for (int l = g - 1; l >= c; --l) ascend(l);
   }
   for (int l = c - 1; l >= 0; --l) ascend(l);
@@ -1540,7 +1527,7 @@ int mg_time_kernels(MGHier *h, int reps, double ms[10]) {
             hipLaunchKernelGGL(k_mg_tail, dim3(1), dim3(kTailThreads), h->tail_lds, stream(), h->tailimg, h->tail,
                                h->nu1, h->nu2, h->coarse_sweeps, nullptr);
           else
-            hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(1024), 0, stream(), h->L[nl - 1], h->coarse_sweeps, nullptr);
+            coarse_solve(h->L[nl - 1], h->coarse_sweeps, nullptr);
           return MOONS_OK;
         case 4: return mg_vcycle(h, nullptr);
         default: return MOONS_OK;
