@@ -331,19 +331,6 @@ __global__ void __launch_bounds__(256) k_apply_bcs(BcArgs A, int implicit_, cons
   }
 }
 
-// Assigns val to one whole plane idx along direction d.
-__global__ void __launch_bounds__(256) k_assign_plane(double *u, Shape3 S, int d, int idx, double val,
-                                                      const int *gate) {
-  if (gate && *gate) return;
-  const int a = (d + 1) % 3, b = (d + 2) % 3;
-  const int na = S.s[a], nb = S.s[b];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= na * nb) return;
-  int ii[3];
-  ii[a] = t % na; ii[b] = t / na; ii[d] = idx;
-  u[idx3(S.s, ii[0], ii[1], ii[2])] = val;
-}
-
 // Assigns val to the ghost planes of the faces in mask (bit f: face f = 2d +
 // side, plane 0 or s_d - 1) in one launch: thread t walks the faces' planes
 // one after another.  Edges shared by two faces get the same value twice.
@@ -374,20 +361,6 @@ static int launch_assign_faces(moons_field_s *u, int mask, double val) {
                      g_gate);
   MOONS_LAUNCH_CHECK();
   return MOONS_OK;
-}
-
-// Multiplies one whole plane idx along direction d by val.
-__global__ void __launch_bounds__(256) k_scale_plane(double *u, Shape3 S, int d, int idx, double val,
-                                                     const int *gate) {
-  if (gate && *gate) return;
-  const int a = (d + 1) % 3, b = (d + 2) % 3;
-  const int na = S.s[a], nb = S.s[b];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= na * nb) return;
-  int ii[3];
-  ii[a] = t % na; ii[b] = t / na; ii[d] = idx;
-  const size_t q = idx3(S.s, ii[0], ii[1], ii[2]);
-  u[q] = u[q] * val;
 }
 
 // del along dir for every output element of the padded range, one thread per
@@ -610,22 +583,6 @@ int launch_assign_ghost_xperiodic(moons_field_s *u, double val) {
     if (!(u->has_bcs && u->bct[face] == MOONS_BC_PERIODIC)) mask |= 1 << face;
   return launch_assign_faces(u, mask, val);
 }
-
-static int launch_plane(moons_field_s *u, int d, int idx, double val, bool scale) {
-  if (d < 0 || d > 2 || idx < 0 || idx >= u->s[d]) return fail(MOONS_ERR_ARG, "plane index out of range");
-  Shape3 S{{u->s[0], u->s[1], u->s[2]}};
-  const int a = (d + 1) % 3, bb = (d + 2) % 3;
-  const size_t np = (size_t)u->s[a] * u->s[bb];
-  if (scale)
-    hipLaunchKernelGGL(k_scale_plane, dim3(nblk(np)), dim3(256), 0, g_stream, u->d, S, d, idx, val, g_gate);
-  else
-    hipLaunchKernelGGL(k_assign_plane, dim3(nblk(np)), dim3(256), 0, g_stream, u->d, S, d, idx, val, g_gate);
-  MOONS_LAUNCH_CHECK();
-  return MOONS_OK;
-}
-
-int launch_plane_set(moons_field_s *u, int d, int idx, double val) { return launch_plane(u, d, idx, val, false); }
-int launch_plane_scale(moons_field_s *u, int d, int idx, double val) { return launch_plane(u, d, idx, val, true); }
 
 int launch_del(moons_field_s *out, const moons_field_s *f, int n, int dir, int pad, int gen) {
   if (dir < 0 || dir > 2 || (n != 1 && n != 2) || gen < 1 || gen > 3 || pad < 0 || pad > 1)

@@ -13,8 +13,7 @@
 //   compute_J, compute_Btot (finite_Rem = F: Btot = B0), compute_JCrossB
 //                              solvers/induction/induction_aux.f90:80-88,
 //                              solvers/induction/induction_sources.f90:70-84
-// Every operator is a device kernel of this library; element-wise chains are
-// fused into one kernel each, keeping the reference's operation order (AB2 =
+// The sources are one kernel a term group (sources.hip), keeping the reference's operation order (AB2 =
 // 1.5 F, then + (-0.5) Fnm1, + L, * dt; Dirichlet wall planes zeroed; + X), so
 // each value is rounded exactly as in the sequential passes.  The fluid and
 // induction meshes are the same single block, so embedding and extraction
@@ -468,7 +467,7 @@ int moons_mhd_field(moons_mhd_t S, int which, moons_field_t out[6]) {
 
 // ---------------------------------------------------------------------------
 // The energy equation: sources (advection, diffusion) and one of the three
-// time-marching methods of solve_energy, composed from the kernels above.
+// time-marching methods of solve_energy.
 // ---------------------------------------------------------------------------
 
 struct moons_nrg_s {
