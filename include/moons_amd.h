@@ -339,7 +339,14 @@ int moons_volume(moons_field_t vol);
 int moons_pcg_sf_create(moons_mesh_t m, int op, int prec, moons_field_t x, moons_pcg_t *out);
 int moons_pcg_destroy(moons_pcg_t pcg);
 /* init(ISP, iter_max, tol_rel, tol_abs, n_skip_check_res, ...)
- * (code/handwritten/var_set/iter_solver_params_extend.f90:44-58). */
+ * (code/handwritten/var_set/iter_solver_params_extend.f90:44-58).  A solve ends
+ * where a tolerance is met or at iter_max.  One exception: a MOONS_PREC_MG_FP32
+ * solver whose hierarchy smooths lines of more than 128 cells (moons_pcg_set_mg)
+ * goes on to a twentieth of the tolerances, because such lines leave a larger
+ * error at the same residual; for as many iterations again as it took to meet a
+ * tolerance (8 if that is more) at most, and still reporting the caller's
+ * tolerances: where iter_max ends it on the way with a tolerance met, exit_loop
+ * has that tolerance's bit and not iter_max's. */
 int moons_pcg_set_isp(moons_pcg_t pcg, int iter_max, double tol_rel, double tol_abs,
                       int n_skip_check_res);
 /* The k of an nrg_diffusion solver: init(PCG%k, k) of init_PCG_SF
@@ -410,8 +417,8 @@ int moons_clean_div_fft(moons_fft_t fft, moons_field_t X[3], moons_field_t Xstar
  * hierarchy): at most max_levels levels, nu1/nu2 smoothing sweeps before/after
  * the coarse correction, coarse_sweeps sweeps on the coarsest level.  A sweep
  * is red-black Gauss-Seidel, or on a level of more than 32^3 cells whose
- * non-periodic y or z cell widths vary by more than 1.5x (lines of at most 128
- * cells), zebra line Gauss-Seidel along those directions: y-lines of both
+ * non-periodic y or z cell widths vary by more than 1.5x (lines of at most 256
+ * cells; the coarsest level is always swept red-black), zebra line Gauss-Seidel along those directions: y-lines of both
  * colours, then z-lines (reversed after the correction).  Defaults 16, 2, 2,
  * 16.  No reference counterpart (see MOONS_PREC_MG_FP32). */
 int moons_pcg_set_mg(moons_pcg_t pcg, int max_levels, int nu1, int nu2, int coarse_sweeps);

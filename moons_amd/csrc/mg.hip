@@ -1467,16 +1467,19 @@ int mg_vcycle(MGHier *h, const int *done) {
   return MOONS_OK;
 }
 
-// The share of the solver's relative tolerance that a solve with this
-// preconditioner goes on to.  Lines longer than 128 cells take out the rough
+// The share of the solver's tolerances that a solve with this preconditioner
+// goes on to (exit_decision, pcg.hip, bounds how long).  Lines longer than 128 cells take out the rough
 // part of the error, which the residual weighs most, so that at one residual
 // the error left is up to 14 times the one that point sweeps leave (14 grids
 // with 136 to 192 cells along y or z: 0.5 to 14 times at 1e-8).  A tenth of the
 // tolerance still leaves 0.05 to 1.4 times it; a twentieth, 2 to 6 iterations
-// more than the tolerance itself, less than it on every one of them.
-double mg_stop_factor(const MGHier *h) {
-  for (const LevelDev &L : h->L)
+// more than the tolerance itself, less than it on every one of them.  The
+// coarsest level is swept by points whatever its shape.
+double mg_stop_share(const MGHier *h) {
+  for (size_t l = 0; l + 1 < h->L.size(); ++l) {
+    const LevelDev &L = h->L[l];
     if ((L.line1 && L.n1 > 128) || (L.line2 && L.n2 > 128)) return 0.05;
+  }
   return 1.0;
 }
 

@@ -27,9 +27,9 @@ void mg_f32_map(const MGHier *h, int map[3]);
 // One V-cycle x0 = V f0 on the library stream; every kernel returns at once
 // when *done (device) is non-zero.
 int mg_vcycle(MGHier *h, const int *done);
-// The share of the relative tolerance a solve goes on to (1, or less where the
-// smoother leaves more error at the same residual).
-double mg_stop_factor(const MGHier *h);
+// The share of its tolerances a solve goes on to (1, or less where the smoother
+// leaves more error at the same residual).
+double mg_stop_share(const MGHier *h);
 // Start of a solve (the learned level's cycle count restarts).
 void mg_begin_solve(MGHier *h);
 // The learned initial guess in the first `cycles` V-cycles of each solve (0: every cycle).

@@ -44,8 +44,9 @@ namespace moons {
 struct PcgCtrl {
   int iter, done, exit_loop, iter_max, n_skip;
   int given_up; // the resident loop was given up (pcg_resident.hpp)
+  int met;      // the iteration that first met a tolerance (multigrid; 0: none yet)
   double tol_rel, tol_abs;
-  double tol_stop; // the relative residual the loop goes on to: tol_rel, or less (mg_stop_factor)
+  double share; // the share of the tolerances the loop goes on to (exit_decision)
   double rho[2]; // rho of the last iteration, indexed by its parity
   double alpha, beta, res0, res, mean, volsum, pq, rr, rz;
 };
@@ -316,23 +317,36 @@ __global__ void __launch_bounds__(kNT) k_pcg_update(double *__restrict__ x, cons
 
 // Exit decision after the x/r update of iteration `it` (check_res every
 // n_skip, update_exit_loop: hw/var_set/iter_solver_params_extend.f90:86-113).
+// A solve ends where a tolerance is met, unless ctrl->share is below 1
+// (mg_stop_share): then it goes on to that share of the tolerance, for as many
+// iterations again as it took to meet it at most, or kTightLeast if that is
+// more, and it ends with the tolerance met.  At a fixed rate of convergence a
+// twentieth of 1e-8 takes a sixth of the iterations again; the limit is for
+// tolerances that the residual meets and then hardly passes.  iter_max reached
+// on the way is no failure: with the tolerance met its flag stays away.
+// met: the iteration that first met a tolerance, so far (0: none).
+constexpr int kTightLeast = 8;
 struct ExitDecision {
   bool stop, checked;
-  int flags;
+  int flags, met;
   double res;
 };
 
-__device__ __forceinline__ ExitDecision exit_decision(const PcgCtrl *ctrl, int it, double rr) {
-  ExitDecision e{false, false, 0, 0.0};
+__device__ __forceinline__ ExitDecision exit_decision(const PcgCtrl *ctrl, int it, double rr, int met = 0) {
+  ExitDecision e{false, false, 0, met, 0.0};
+  const bool last = it >= ctrl->iter_max;
   if (it % ctrl->n_skip == 0) {
     e.checked = true;
     e.res = sqrt(fabs(rr));
-    const bool e1 = e.res / ctrl->res0 < ctrl->tol_rel, e2 = e.res < ctrl->tol_abs, e3 = it >= ctrl->iter_max;
-    e.flags = (e1 ? 1 : 0) | (e2 ? 2 : 0) | (e3 ? 4 : 0);
-    e.stop = e.res / ctrl->res0 < ctrl->tol_stop || e2 || e3;
-  }
-  if (!e.stop && it >= ctrl->iter_max) {
-    e.flags |= 4;
+    const double rel = e.res / ctrl->res0;
+    const bool e1 = rel < ctrl->tol_rel, e2 = e.res < ctrl->tol_abs;
+    const bool tight = rel < ctrl->tol_rel * ctrl->share || e.res < ctrl->tol_abs * ctrl->share;
+    if ((e1 || e2) && !met) e.met = it;
+    const bool enough = (e1 || e2) && it - e.met >= max(kTightLeast, e.met);
+    e.flags = (e1 ? 1 : 0) | (e2 ? 2 : 0) | (last && !(met && (e1 || e2)) ? 4 : 0);
+    e.stop = tight || enough || last;
+  } else if (last) {
+    e.flags = met && (ctrl->exit_loop & 3) ? 0 : 4;
     e.stop = true;
   }
   return e;
@@ -415,8 +429,10 @@ __global__ void __launch_bounds__(kNT) k_pcg_check(PcgCtrl *ctrl, const double *
   if (ctrl->done) return;
   __shared__ double sh[kNT / kWave];
   const double rr = prologue_sum<kNT>(partB, nb, 2, 0, sh);
-  const ExitDecision e = exit_decision(ctrl, it, rr);
-  if (threadIdx.x == 0) publish_exit(ctrl, it, rr, e);
+  if (threadIdx.x != 0) return;
+  const ExitDecision e = exit_decision(ctrl, it, rr, ctrl->met);
+  ctrl->met = e.met;
+  publish_exit(ctrl, it, rr, e);
 }
 
 // Partials of (z,r) and (z,q) with z the V-cycle output.
@@ -651,18 +667,19 @@ __global__ void k_pcg_ctrl_set(PcgCtrl *ctrl, int iter_max, int n_skip, double t
                                double volsum) {
   if (threadIdx.x != 0) return;
   PcgCtrl h;
-  h.iter = h.done = h.exit_loop = h.given_up = 0;
+  h.iter = h.done = h.exit_loop = h.given_up = h.met = 0;
   h.iter_max = iter_max;
   h.n_skip = n_skip;
-  h.tol_rel = h.tol_stop = tol_rel;
+  h.tol_rel = tol_rel;
   h.tol_abs = tol_abs;
+  h.share = 1.0;
   h.rho[0] = h.rho[1] = 0.0;
   h.alpha = h.beta = h.res0 = h.res = h.mean = h.pq = h.rr = h.rz = 0.0;
   h.volsum = volsum;
   *ctrl = h;
 }
 
-static double tol_stop(const moons_pcg_s *S) { return S->tol_rel * (S->mg ? mg_stop_factor(S->mg) : 1.0); }
+static double stop_share(const moons_pcg_s *S) { return S->mg ? mg_stop_share(S->mg) : 1.0; }
 
 // The initial control block lives in its own pinned buffer, written only
 // here, so a captured copy of it replays the same values.
@@ -678,8 +695,8 @@ static int pcg_upload_ctrl(moons_pcg_s *S) {
   h.iter_max = S->iter_max;
   h.n_skip = S->n_skip;
   h.tol_rel = S->tol_rel;
-  h.tol_stop = tol_stop(S);
   h.tol_abs = S->tol_abs;
+  h.share = stop_share(S);
   h.volsum = S->volsum;
   if (std::memcmp(&h, S->host_init, sizeof(PcgCtrl)) != 0) {
     // a copy of the old contents may still be pending
@@ -1113,7 +1130,7 @@ static int pcg_solve_impl(moons_pcg_s *S, moons_field_t x, moons_field_t b) {
       tail_pending = false;
     }
     int chunk = launched == 0 ? (mg ? 3 : 16)
-                              : next_chunk(*S->host_ctrl, tol_stop(S), mg ? 1 : 4, mg ? 32 : 512);
+                              : next_chunk(*S->host_ctrl, S->tol_rel * stop_share(S), mg ? 1 : 4, mg ? 32 : 512);
     chunk = std::min(chunk, S->iter_max - launched);
     for (int c = 0; c < chunk; ++c) {
       const int it = launched + c + 1;

@@ -257,6 +257,90 @@ def test_vcycle_long_lines_match_restatement(gpu, monkeypatch, case):
     assert err < 4 * own, (err, own)
 
 
+def expected_stop(res, isp, share):
+    """Iterations and exit flags of a solve whose residual after n iterations is res[n]: it ends where a tolerance is
+    met (share 1), or goes on to `share` of it, at most for max(8, the iterations so far) more, with the tolerance met."""
+    iter_max, tol_rel, tol_abs, n_skip = isp
+    met = flags = 0
+    for it in range(1, iter_max + 1):
+        last = it == iter_max
+        if it % n_skip:
+            if last:
+                return it, flags | (0 if met and flags & 3 else 4), met
+            continue
+        rel = res[it] / res[0]
+        ok = (rel < tol_rel, res[it] < tol_abs)
+        flags = ok[0] + 2 * ok[1] + (4 if last and not (met and any(ok)) else 0)
+        if any(ok) and not met:
+            met = it
+        if (rel < tol_rel * share or res[it] < tol_abs * share or last
+                or (any(ok) and it - met >= max(8, met))):
+            return it, flags, met
+
+
+LONG_STOP = {  # (max_levels, nu1, nu2, coarse sweeps), the share of the tolerances it goes on to
+    "long_lines": ((16, 2, 2, 16), 0.05),
+    "long_lines_weak_cycle": ((2, 1, 1, 1), 0.05),
+    "one_level_of_points": ((1, 2, 2, 16), 1.0),
+}
+
+
+@pytest.mark.parametrize("case", list(LONG_STOP))
+def test_stop_of_a_solve_with_long_lines(gpu, case):
+    """Where a mixed solve on a 16 x 136 x 16 stretched grid ends and what it reports, against its own residuals: each
+    tolerance, a check every third iteration, iter_max between the tolerance and the share, and a tolerance whose share
+    is far (the weak cycle).  A hierarchy of one level smooths no lines and stops at the tolerance."""
+    mg, share = LONG_STOP[case]
+    hs = [O.uniform_nodes(0.0, 1.0, 16), O.roberts_both_nodes(0.0, 1.0, 136, 1.05), O.uniform_nodes(0.0, 1.0, 16)]
+    m = gpu.mesh(*hs)
+    X = gpu.SF(m, "CC").set_BCs(["Neumann"] * 6, None, all_Neumann=True)
+    B = gpu.SF(m, "CC").upload(np.asfortranarray(np.random.default_rng(6).standard_normal(m.shape(0))))
+    P = mg_solver(gpu, m, X)
+    P.set_MG(*mg)
+
+    def solve(*isp):
+        X.fill(0.0)
+        P.set_ISP(gpu.iter_solver_params(*isp))
+        return P.solve(X, B)
+
+    n = 60
+    infos = [solve(q, 1e-300, 1e-300, 1) for q in range(1, n + 1)]
+    res = [infos[0].res_norm0] + [i.res_norm for i in infos]
+    tol = 1.0001 * min(res[1:4]) / res[0] if mg[0] < 16 else 1e-6
+    first = next(q for q in range(1, n) if res[q] / res[0] < tol)
+    ends = []
+    for isp in [(n, tol, 1e-300, 1), (n, 1e-300, tol * res[0], 1), (first + 1, tol, 1e-300, 1), (n, tol, 1e-300, 3),
+                (3 * ((first + 2) // 3) + 1, tol, 1e-300, 3)]:
+        info = solve(*isp)
+        print(f"stop {case} {isp}: {info.iterations} {info.exit_loop}", flush=True)
+        ends.append((info.iterations, info.exit_loop))
+        assert ends[-1] == expected_stop(res, isp, share)[:2], isp
+    # the first stop, and why: the share is reached, or (weak cycle) the limit, or the tolerance itself
+    it, flags = ends[0]
+    assert flags == 1
+    assert {"long_lines": res[it] / res[0] < 0.05 * tol, "long_lines_weak_cycle": it == first + 8,
+            "one_level_of_points": it == first}[case]
+    assert ends[2][1] == 1  # iter_max with the tolerance met
+
+
+def test_solution_of_a_solve_with_long_lines(gpu):
+    """The solution of a 1e-8 solve on lines of 136 cells within the 1e-6 stated for mixed-precision fields."""
+    hs = [O.uniform_nodes(0.0, 1.0, 16), O.roberts_both_nodes(0.0, 1.0, 136, 1.05), O.uniform_nodes(0.0, 1.0, 16)]
+    g, m = O.Grid(*hs), gpu.mesh(*hs)
+    types = ["Neumann"] * 6
+    b = np.asfortranarray(O.splitmix(int(np.prod(g.shape(0))), 29).reshape(g.shape(0), order="F"))
+    xr = np.zeros(g.shape(0), order="F")
+    O.pcg_lap(g, 0, O.BCs.make(types), True, xr, b, 20000, 1e-13, 1e-300)
+    X = gpu.SF(m, "CC").set_BCs(types, None, all_Neumann=True)
+    info = mg_solver(gpu, m, X).solve(X, gpu.SF(m, "CC").upload(b))
+    assert info.exit_loop == 1
+    vi = O.volume(g, 0)[1:-1, 1:-1, 1:-1]
+    x, xr = (a[1:-1, 1:-1, 1:-1] - (a[1:-1, 1:-1, 1:-1] * vi).sum() / vi.sum() for a in (X.download(), xr))
+    err = np.linalg.norm(x - xr) / np.linalg.norm(xr)
+    print(f"long lines solve: {info.iterations} iterations, error {err:.2e}", flush=True)
+    assert err < 1e-6, err
+
+
 @pytest.mark.parametrize("case", list(CASES))
 def test_mixed_pcg_matches_fp64_oracle(gpu, case):
     N, beta, bct = CASES[case]
