@@ -360,6 +360,12 @@ int moons_pcg_sf_update_mfp(moons_pcg_t pcg, double coeff_implicit_time_split, i
  * b the right-hand side, both device fields of the solver's location.  The
  * whole loop runs on the device; info may be NULL. */
 int moons_pcg_sf_solve(moons_pcg_t pcg, moons_field_t x, moons_field_t b, moons_pcg_info *info);
+/* How the solver's Jacobi solves run: planes and blocks of the loop that stays
+ * resident on the GPU (planes a thread, workgroups; both 0 where each iteration
+ * is launched), and given_up, 1 once its workgroups were not all resident
+ * together (the solve was then redone, and later ones are, by launches).  Any
+ * pointer may be NULL.  No reference counterpart. */
+int moons_pcg_resident(moons_pcg_t pcg, int *planes, int *blocks, int *given_up);
 /* The PPE solve of moons_pcg_sf_solve (Lap_uniform_SF with prec_Lap_SF, FP64
  * Jacobi-PCG, ISP as moons_pcg_set_isp) without a solver object and without
  * allocating: no counterpart in the reference; it is for callers that cannot

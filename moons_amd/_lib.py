@@ -124,6 +124,7 @@ SIGNATURES = {
                                       C.c_void_p]),
     "moons_pcg_set_mg": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int]),
     "moons_pcg_mg_info": (C.c_int, [C.c_void_p, c_int_p, c_int_p]),
+    "moons_pcg_resident": (C.c_int, [C.c_void_p, c_int_p, c_int_p, c_int_p]),
     "moons_pcg_apply_prec": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]),
     "moons_pcg_vf_create": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p),
                                       C.POINTER(C.c_void_p)]),

@@ -449,6 +449,12 @@ class PCG_solver_SF:
         check(load().moons_pcg_mg_info(self.handle, C.byref(lv), n))
         return lv.value, (n[0], n[1], n[2])
 
+    def resident(self):
+        """(planes a thread, workgroups, given up) of the resident Jacobi loop; (0, 0, ...) where iterations are launched."""
+        v = [C.c_int() for _ in range(3)]
+        check(load().moons_pcg_resident(self.handle, *[C.byref(q) for q in v]))
+        return tuple(q.value for q in v)
+
     def set_MG_UNet(self, net: "UNet | None", level: int = 2, cycles: int = 0) -> None:
         """Learned initial guess of multigrid level `level` inside the V-cycle
         (prec="MG_FP32"), in the first `cycles` V-cycles of each solve (0: every one)."""

@@ -640,7 +640,8 @@ struct moons_pcg_s {
   ResPlan res;                  // the resident loop's box (cpt 0: the launch-per-kernel loop)
   unsigned long long *slots = nullptr;
   double *part63 = nullptr;     // the boxes' block sums (3 a box), beside the slots
-  int spins = 0;                // its waits' bound
+  int spins = 0;                // its waits' bound, in looks at a slot
+  int given_up = 0;             // its waits were given up once: launched loop from then on
   bool noalloc = false;         // a one-shot solver over the static scratch (no host_init)
 };
 
@@ -743,10 +744,13 @@ static const void *resident_kernel(const ResPlan &P, int op) {
 }
 
 // Chooses the resident loop's box for S (Jacobi solves of a grid that fits the
-// GPU's CUs), or none.  MOONS_RESIDENT_SPINS sets the bound of its waits (0:
+// GPU's CUs), or none.  A wait looks at its slot 2^16 times at most: 0.15 us a
+// look, 10 ms, the time of hundreds of iterations (5 to 16 us each), far beyond
+// the time a block of another stream's kernel holds its CU.  It is paid once a
+// solver at most (pcg_solve_impl).  MOONS_RESIDENT_SPINS sets another bound (0:
 // the launch-per-kernel loop), for tests of both loops and of the give-up path.
 static void resident_setup(moons_pcg_s *S) {
-  S->spins = 1 << 20;
+  S->spins = 1 << 16;
   if (const char *e = getenv("MOONS_RESIDENT_SPINS")) S->spins = atoi(e);
   if (S->spins <= 0) return;
   for (int d = 0; d < 3; ++d) // a periodic face has its partner
@@ -1086,12 +1090,13 @@ static int pcg_solve_impl(moons_pcg_s *S, moons_field_t x, moons_field_t b) {
     if (resident) {
       if ((st = pcg_solve_resident(S, x))) return st;
       if (!S->host_ctrl->given_up) return MOONS_OK;
-      // not every block was resident: the solve again from x, a kernel at a time
-      const ResPlan keep = S->res;
+      // Not every block was resident: the solve again from x, a kernel at a
+      // time, and so are this solver's later ones (eager and captured), which
+      // would otherwise wait out the bound each time on a GPU whose CUs are
+      // masked or shared with another process's resident loop.
       S->res.cpt = 0;
-      st = pcg_solve_impl(S, x, b);
-      S->res = keep;
-      return st;
+      S->given_up = 1;
+      return pcg_solve_impl(S, x, b);
     }
   } else {
     // z0 = V(r0/vol), rho0 = (z0,r0), p = z0
@@ -1292,6 +1297,14 @@ int moons_pcg_mg_info(moons_pcg_t S, int *levels, int n_coarsest[3]) {
   const int nl = mg_levels(S->mg);
   if (levels) *levels = nl;
   if (n_coarsest) mg_level_cells(S->mg, nl - 1, n_coarsest);
+  return MOONS_OK;
+}
+
+int moons_pcg_resident(moons_pcg_t S, int *planes, int *blocks, int *given_up) {
+  if (!S) return fail(MOONS_ERR_ARG, "moons_pcg_resident: null solver");
+  if (planes) *planes = S->res.cpt;
+  if (blocks) *blocks = S->res.cpt ? S->res.nb() : 0;
+  if (given_up) *given_up = S->given_up;
   return MOONS_OK;
 }
 

@@ -40,7 +40,8 @@
 // all be resident, every wait is bounded: a block that gives up sets `abort`,
 // the others see it while they wait, every block returns, x is untouched (the
 // result goes to a buffer that k_pcg_take copies only from a complete run),
-// and the host solves again with the launch-per-kernel loop.
+// and the host solves again with the launch-per-kernel loop, and with it only
+// from then on.
 #pragma once
 
 namespace moons {
