@@ -158,6 +158,41 @@ def test_forward_and_gradients_exact(gpu, shape, seed, pc):
         off += n
 
 
+def exact_net(w):
+    """The float64 restatement, which fails where BF16 storage would round a value."""
+    net = UO.Net(w, bf=False)
+
+    def kept(x):
+        np.testing.assert_array_equal(UO.bf16(x), x)
+        return x
+
+    net.r = kept
+    return net
+
+
+def padded_sample(xi, ti):
+    """(n2, n1, n0, 4) input and (n2, n1, n0) target as the host arrays the network takes."""
+    x = np.zeros((4,) + tuple(n + 2 for n in ti.shape[::-1]), dtype=np.float32)
+    x[:, 1:-1, 1:-1, 1:-1] = np.transpose(xi, (3, 2, 1, 0))
+    t = np.zeros(x.shape[1:], dtype=np.float32)
+    t[1:-1, 1:-1, 1:-1] = np.transpose(ti, (2, 1, 0))
+    return x, t
+
+
+# below and above the size at which the output layer runs as LDS tiles, the tiles ragged along x
+@pytest.mark.parametrize("shape", [(36, 36, 36), (36, 40, 36)])
+def test_forward_exact_around_the_output_tiles(gpu, shape):
+    print(f"unet exact forward {shape}", flush=True)
+    w = exact_weights(1, 0.8)
+    n0, n1, n2 = shape
+    xi = np.random.default_rng(7).integers(1, 3, (n2, n1, n0, 4)).astype(np.float64)
+    ref = exact_net(w).forward(xi)
+    net = gpu.UNet(seed=0)
+    net.set_weights(w.astype(np.float32))
+    out = net.forward(padded_sample(xi, ref)[0])[1:-1, 1:-1, 1:-1]
+    np.testing.assert_array_equal(out.astype(np.float64), UO.from_internal(ref))
+
+
 def test_training_lowers_the_loss(gpu):
     print("unet training", flush=True)
     from moons_amd import learned
