@@ -193,6 +193,36 @@ def test_forward_exact_around_the_output_tiles(gpu, shape):
     np.testing.assert_array_equal(out.astype(np.float64), UO.from_internal(ref))
 
 
+def test_forward_and_gradients_exact_second_level_tiles(gpu):
+    """As test_forward_and_gradients_exact, at 32 x 64 x 64: the smallest size whose second level (16 x 32 x 32, 256
+    tiles) runs through the LDS-tiled kernels, forward and data gradients of the 16 -> 32 and 32 -> 32 layers."""
+    shape = (32, 64, 64)
+    print(f"unet exact {shape}", flush=True)
+    w = exact_weights(1, 0.8)
+    rng = np.random.default_rng(101)
+    n0, n1, n2 = shape
+    xi = rng.integers(1, 3, (n2, n1, n0, 4)).astype(np.float64)
+    ref = exact_net(w)
+    out0 = ref.forward(xi)
+    # one voxel in ten off its target, so that the sums of the gradients stay exact
+    d = rng.integers(-1, 2, (n2, n1, n0)) * 0.25 * (rng.random((n2, n1, n0)) < 0.1)
+    rg = UO.pack(ref.backward(2.0 * d / d.size))
+    assert np.array_equal(rg.astype(np.float32).astype(np.float64), rg)
+    net = gpu.UNet(seed=0)
+    net.set_weights(w.astype(np.float32))
+    x, t = padded_sample(xi, out0 - d)
+    out = net.forward(x)[1:-1, 1:-1, 1:-1]
+    np.testing.assert_array_equal(out.astype(np.float64), UO.from_internal(out0))
+    loss, g = net.grad(x, t)
+    assert loss == (d * d).sum() / d.size
+    np.testing.assert_array_equal(g.astype(np.float64), rg)
+    off = 0
+    for ci, co in UO.LAYERS:
+        n = 27 * ci * co + co
+        assert np.count_nonzero(rg[off:off + n]) > 0
+        off += n
+
+
 def test_training_lowers_the_loss(gpu):
     print("unet training", flush=True)
     from moons_amd import learned
