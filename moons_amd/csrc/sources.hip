@@ -571,7 +571,7 @@ bool edges_fit(moons_field_s *const E[3], moons_field_s *const U_E[6], moons_fie
         if (f[q]->d == f[r]->d && (q >= 3 || r == 0)) return false; // an operand that is also a result
     }
   }
-  return true;
+  return !current_gate();
 }
 
 int launch_edge_cross(moons_field_s *const E[3], moons_field_s *const U_E[6], moons_field_s *const B[3],

@@ -757,7 +757,6 @@ __global__ void __launch_bounds__(kUT) k_pack32(const float *W, int Cin, int Cou
   WB[t] = r;
 }
 
-// BF16-rounded FP32 copy of the small layers' weights (the values the network uses)
 // first layer (k_conv_in): step s, lane: k = 32 s + 8 (lane / 16) ..+8 of the
 // 27 x 4 (tap, channel) pairs, zeros past them
 __global__ void __launch_bounds__(kUT) k_pack_in(const float *W, u16x8 *WB) {
@@ -771,6 +770,7 @@ __global__ void __launch_bounds__(kUT) k_pack_in(const float *W, u16x8 *WB) {
   WB[threadIdx.x] = r;
 }
 
+// BF16-rounded FP32 copy of the small layers' weights (the values the network uses)
 __global__ void __launch_bounds__(kUT) k_round_bf16(const float *W, float *Wr, size_t n) {
   const size_t t = (size_t)blockIdx.x * kUT + threadIdx.x;
   if (t < n) Wr[t] = bf2f(f2bf(W[t]));
