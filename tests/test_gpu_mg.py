@@ -257,6 +257,61 @@ def test_vcycle_long_lines_match_restatement(gpu, monkeypatch, case):
     assert err < 4 * own, (err, own)
 
 
+COARSE = {  # cells, BCs, levels: a coarsest level beyond the LDS tail, by fused sweeps or (above 64^3 cells) half-sweeps
+    "one_level_fused": ((50, 39, 45), [2, 1, 2, 2, 1, 2], 1),
+    "one_level_half_sweeps": ((65, 65, 63), [2, 2, 2, 2, 2, 2], 1),
+    "second_of_two_levels": ((90, 70, 50), [2, 2, 1, 2, 2, 2], 2),
+}
+
+
+@pytest.mark.parametrize("sweeps", [16, 5])
+@pytest.mark.parametrize("case", list(COARSE))
+def test_vcycle_large_coarsest_level_matches_restatement(gpu, case, sweeps):
+    """A coarsest level too large for the LDS tail, where an odd count ends coarsening early: even and odd sweep counts
+    (a fused sweep swaps the level's two buffers) against the restatement, and the same bits from a second cycle."""
+    n, bct, nl = COARSE[case]
+    print(f"vcycle coarse end {case} {sweeps}", flush=True)
+    hs = [O.uniform_nodes(0.0, 1.0, n[0])] + [O.roberts_both_nodes(0.0, 1.0, q, 1.1) for q in n[1:]]
+    g, m = O.Grid(*hs), gpu.mesh(*hs)
+    levels = MGO.build(hs, bct)
+    assert len(levels) == nl
+    x = gpu.SF(m, "CC").set_BCs([NAMES[t] for t in bct], None, all_Neumann=(1 not in bct))
+    P = mg_solver(gpu, m, x)
+    P.set_MG(16, 2, 2, sweeps)
+    assert P.mg_info() == (nl, tuple(levels[-1].n))
+    r = np.zeros(g.shape(0), order="F")
+    r[1:-1, 1:-1, 1:-1] = np.random.default_rng(23).standard_normal(n)
+    R, Z, Z2 = gpu.SF(m, "CC").upload(r), gpu.SF(m, "CC"), gpu.SF(m, "CC")
+    P.apply_prec(R, Z)
+    P.apply_prec(R, Z2)
+    np.testing.assert_array_equal(Z2.download(), Z.download())
+    vol = O.volume(g, 0)
+    f = np.zeros(g.shape(0))
+    f[1:-1, 1:-1, 1:-1] = r[1:-1, 1:-1, 1:-1] / vol[1:-1, 1:-1, 1:-1]
+    z, zr = (a[1:-1, 1:-1, 1:-1] for a in (Z.download(), MGO.vcycle(levels, f, bct, coarse_sweeps=sweeps)))
+    err = np.linalg.norm(z - zr) / np.linalg.norm(zr)
+    assert err < 2e-5, err
+
+
+@pytest.mark.parametrize("sweeps", [16, 5])
+def test_solve_on_a_single_level_of_points(gpu, sweeps):
+    """The PCG around that cycle, whose result lies in either buffer, against the converged FP64 solution."""
+    n, bct, _ = COARSE["one_level_fused"]
+    hs = [O.uniform_nodes(0.0, 1.0, n[0])] + [O.roberts_both_nodes(0.0, 1.0, q, 1.1) for q in n[1:]]
+    g, m = O.Grid(*hs), gpu.mesh(*hs)
+    types = [NAMES[t] for t in bct]
+    b = np.asfortranarray(O.splitmix(int(np.prod(g.shape(0))), 31).reshape(g.shape(0), order="F"))
+    xr = np.zeros(g.shape(0), order="F")
+    O.pcg_lap(g, 0, O.BCs.make(types), False, xr, b, 20000, 1e-13, 1e-300)
+    X = gpu.SF(m, "CC").set_BCs(types, None)
+    P = mg_solver(gpu, m, X, iters=1000, tol=1e-10)
+    P.set_MG(16, 2, 2, sweeps)
+    info = P.solve(X, gpu.SF(m, "CC").upload(b))
+    err = np.linalg.norm((X.download() - xr)[1:-1, 1:-1, 1:-1]) / np.linalg.norm(xr[1:-1, 1:-1, 1:-1])
+    print(f"single level, {sweeps} sweeps: {info.iterations} iterations, error {err:.2e}", flush=True)
+    assert info.exit_loop == 1 and err < 1e-6, (info, err)
+
+
 def expected_stop(res, isp, share):
     """Iterations and exit flags of a solve whose residual after n iterations is res[n]: it ends where a tolerance is
     met (share 1), or goes on to `share` of it, at most for max(8, the iterations so far) more, with the tolerance met."""
