@@ -8,10 +8,10 @@
 // (code/handwritten/solvers/preconditioners/preconditioners.f90:55-71) and
 // modify_RHS_SF (code/handwritten/solvers/PCG/PCG_aux.f90:30-54).
 //
-// A Jacobi solve of a grid that fits the CUs' registers and LDS (up to 128^3)
-// runs its whole loop as one resident kernel (pcg_resident.hpp; in a captured
-// graph as three kernels an iteration over the same blocks, with the same
-// bits).  Otherwise, and in the flexible PCG around the multigrid or the
+// A Jacobi solve of a grid that fits the CUs' registers and LDS (up to 128^3
+// where whole rows fill the blocks, resident_plan) runs its whole loop as one
+// resident kernel (pcg_resident.hpp; in a captured graph as three kernels an
+// iteration over the same blocks, with the same bits).  Otherwise, and in the flexible PCG around the multigrid or the
 // network, one iteration is three HBM-bound kernels over the interior cells:
 //   k_pcg_matvec   q = vol*lap(p), partial (p,q)              read p, write q        16 B/cell
 //   k_pcg_update   x += a p, r -= a q, partials (r,r),(Minv r,r) read x,p,r,q write x,r 48 B/cell

@@ -647,11 +647,12 @@ __global__ void __launch_bounds__(kNT) k_pcg_take(double *__restrict__ x, const 
 // two all-reduces with the halo's loads by the number of blocks (4.5 us to 16
 // blocks, then 1.3 us a doubling to 64, 0.7 us above) and the cells' work by
 // the planes a thread (4 planes 0.8 us, 8 2.4 us, 16 6.5 us).  E.g. 32^3 takes
-// 16 blocks of 4 planes (5.8 us; 64 blocks of 1 plane 7.3 us), 64^3 256 of 2
+// 16 blocks of 4 planes (5.8 us; 64 blocks of 1 plane 7.3 us), 64^3 128 of 4
 // (9.0; 64 of 8 10.1), 128^3 256 of 16 (16.4 us).  The launch-per-kernel loop
 // takes 16-19 us up to 64^3, 32 us at 96^3, 49 us at 128^3, so every grid that
-// fits a box takes the resident one; larger grids, and rows of more than
-// kResNT cells, keep the other.
+// fits a box takes the resident one; the other is kept by larger grids, by rows
+// of more than kResNT cells, and by grids near 128^3 whose rows leave much of a
+// block idle (129 x 128 x 128 and 130 x 120 x 120 need more than 256 blocks).
 constexpr int kResNT = 512;
 inline ResPlan resident_plan(int n0, int n1, int n2, int cus) {
   ResPlan best;
