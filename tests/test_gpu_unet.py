@@ -32,6 +32,22 @@ def test_mfma32_lane_layout(gpu):
     np.testing.assert_array_equal(D, A @ B)
 
 
+# sum, sum of squares, first two and last weight of std::normal_distribution<float> on std::mt19937_64, layer by layer
+INITIAL = {0: (20.117589885353887, 639.63294766430079, "0x1.c67896p-7", "-0x1.0c4984p-4", "-0x1.167f12p-6"),
+           7: (-56.772973754356499, 638.61516517875691, "0x1.e66f9cp-4", "-0x1.0f0d04p-3", "-0x1.6a5adep-7")}
+
+
+@pytest.mark.parametrize("seed", list(INITIAL))
+def test_initial_weights(gpu, seed):
+    w = gpu.UNet(seed=seed).get_weights()
+    W = np.concatenate([a.ravel() for a, _ in UO.unpack(w)])
+    total, squares, *some = INITIAL[seed]
+    assert [W[0], W[1], W[-1]] == [float.fromhex(v) for v in some]
+    # (another order of 355 thousand float64 additions)
+    assert abs(W.sum() - total) < 1e-9 and abs((W * W).sum() - squares) < 1e-9
+    assert not np.concatenate([b for _, b in UO.unpack(w)]).any()
+
+
 def sample_input(shape, seed):
     rng = np.random.default_rng(seed)
     x = np.zeros((4,) + tuple(s + 2 for s in shape), dtype=np.float32)
