@@ -386,8 +386,8 @@ def run_duct(M, args):
 def run_fft(M, args):
     """The cosine-transform direct solver (the reference's FFT pressure path,
     one independent 2D Neumann problem per plane normal to x) at N^3 on a
-    uniform grid, inputs resident in HBM; one step = one solve (pack, DCT-II
-    along y and z as FP64 GEMMs, mode scaling, inverse, unpack, BCs)."""
+    uniform grid, inputs resident in HBM; one step = one solve (DCT-II
+    along y and z as FP64 GEMMs, mode scaling, inverse, BCs)."""
     N = args.fft
     hs = [M.nodes_uniform(0.0, 1.0, N)] * 3
     m = M.mesh(*hs)
@@ -411,7 +411,7 @@ def run_fft(M, args):
                       "transforms": "DCT-II along y and z as FP64 GEMMs (rocBLAS)"},
            "roofline": {"bound": "mfma", "achieved": round(tfs, 2), "peak": 78.6, "unit": "TFLOP/s",
                         "frac": round(tfs / 78.6, 4), "traffic": None,
-                        "flop_per_solve": flop, "note": "whole solve (GEMMs plus pack, scale, unpack, BCs)"}}
+                        "flop_per_solve": flop, "note": "whole solve (GEMMs plus scale, BCs)"}}
     print(json.dumps(out), flush=True)
 
 
