@@ -462,8 +462,9 @@ def run_energy(M, args):
            "last_step_iterations": info["iterations"], "kernels": kern,
            "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": 8000.0, "unit": "GB/s",
                         "frac": round(gbs / 8000.0, 4), "traffic": load_traffic("energy_step_128.md") if N == 128 else None,
-                        "kernel": "nrg_matvec",
-                        "bytes_per_cell": 40}}
+                        "kernel": "nrg_matvec", "bytes_per_cell": 40,
+                        "note": "the launched loop's kernel, back to back; the steps solve in the resident loop"
+                                if P.resident()[0] else "the solve's own kernel, back to back"}}
     # the same step with every source of add_all_energy_sources on (advection,
     # diffusion into L, KE diffusion, viscous dissipation, Joule heating of a
     # seeded J with sigmaInv 1, volumetric heating) and the 3-stage RK with
