@@ -651,7 +651,10 @@ int launch_jxb(moons_field_s *const out[3], moons_field_s *const J[3], moons_fie
 }
 
 int launch_nrg_source(const NrgSource &S) {
-  if (S.T->n >= ((size_t)1 << 31)) return fail(MOONS_ERR_ARG, "fields of 2^31 or more elements are not supported");
+  // (volumetric heating reads its own element alone; elements are numbered in 32 bits)
+  const bool stencils = S.advection || S.diffusion || S.KE || S.viscous || S.joule;
+  if (S.T->n >= (size_t)1 << (stencils ? 31 : 32))
+    return fail(MOONS_ERR_ARG, "fields of 2^31 or more elements are not supported");
   NrgArgs A{};
   const dim3 grid((unsigned)((S.T->n + kSrc - 1) / kSrc));
   const MeshDev &M = S.T->m->dev;

@@ -211,3 +211,27 @@ def test_energy_joule_needs_its_fields(gpu):
         st.step(1)
     with pytest.raises(gpu.MoonsError, match="edge"):
         st.set_joule([gpu.SF(m, "CC").fill(0.0)] * 3, gpu.SF(m, "CC").fill(1.0))
+
+
+@pytest.mark.parametrize("diffusion", [False, True])
+def test_fields_of_more_than_2_31_cells(gpu, diffusion):
+    """A step without a source that reads neighbours takes fields of 2^31 and more cells, every element of them; one
+    with such a source is refused.  (Ten fields of 17 GB on the device.)"""
+    print(f"energy 2^31 cells, diffusion {diffusion}", flush=True)
+    m = gpu.mesh(*[gpu.nodes_uniform(0.0, 1.0, n) for n in (2046, 1022, 1024)])
+    assert np.prod(m.shape(0)) > 2 ** 31
+    try:
+        T = gpu.SF(m, "CC").fill(0.5)
+        st = gpu.Energy_step(m, T, dt=0.125, method=2, advection=(False, 0.0), diffusion=(diffusion, 0.01))
+    except gpu.MoonsError as e:
+        if "hipMalloc" in str(e):
+            pytest.skip("not enough device memory")
+        raise
+    st.field("F").fill(1.0)
+    if diffusion:
+        with pytest.raises(gpu.MoonsError, match="elements are not supported"):
+            st.step(1)
+        return
+    st.step(1)  # T + dt (1.5 0 - 0.5 1)
+    t = T.download()
+    assert t.min() == t.max() == 0.4375
